@@ -10,6 +10,7 @@
 
 #include "aderdg.hpp"
 #include "exa_device.hpp"
+#include "line_ops.hpp"
 
 #include <cfloat>
 #include <type_traits>
@@ -24,11 +25,6 @@ namespace exa {
 // reference's bound, whichever is reached first).
 constexpr double kPicardTol2 = 1e-7 * 1e-7;
 constexpr float kPicardRelTol32 = 1e-6f;
-
-template <typename T>
-__device__ constexpr T tc(double v) {
-  return static_cast<T>(v);
-}
 
 // S = algebraicSource(Q) - NCP(Q, gradQ) at node (z,y,x) of a time slice whose
 // variables are staged in sQ[var][node] (spaceTimePredictorNonlinear.cpph:238-266).
@@ -82,7 +78,7 @@ struct PredictorLayout {
   static constexpr long kLdsBudget = (long)LDSK * 1024;
   static constexpr long kSliceBytes = (long)V * B3 * sizeof(T);
   static constexpr long kOther =
-      (long)(SF + (USE_NCP ? V * B3 : 0) + 2 * B2 + B + 3 + 2 * (NT / kWave)) * sizeof(T);
+      (long)(SF + (USE_NCP ? V * B3 + B2 : 0) + 3 + 2 * (NT / kWave)) * sizeof(T);
   static constexpr long kFree = kLdsBudget - kOther;
   static constexpr int NQL = kFree <= 0 ? 0 : (kFree / kSliceBytes >= B ? B : (int)(kFree / kSliceBytes));
   static constexpr int NQR = B - NQL;
@@ -93,9 +89,11 @@ struct PredictorLayout {
   // (measured: N=4 -2%, N=5 -4% predictor time; at N=6 the rolled form was
   // 19% slower, so N=6 stays unrolled), and the double form of the
   // 5-variable PDE at N=3, where the rolled loop leaves room for the
-  // accumulated time averages (the predictor kernel's ACC_FH).
+  // accumulated time averages (the predictor kernel's ACC_FH), and at N=5,
+  // whose unrolled slices beside the closed first iteration exceed the 256
+  // registers of the two wavefronts per SIMD its LDS allows.
   static constexpr bool ROLLED = (B >= 7 && (IS_FP64 || B >= 8)) || V >= 9 || (!IS_FP64 && (B == 5 || B == 6)) ||
-                                 (IS_FP64 && B == 4 && V == 5);
+                                 (IS_FP64 && (B == 4 || B == 6) && V == 5);
   // 8+ waves per workgroup leave 256 registers per lane, no room for slices;
   // a rolled loop cannot index registers.
   static constexpr bool WSQ = NQR > 0 && (NT >= 8 * kWave || ROLLED);
@@ -148,9 +146,7 @@ __global__ __launch_bounds__(node_threads(B), (predictor_min_waves<B, TERMS, T>(
   __shared__ T sF[SF];
   __shared__ T sQi[NQL > 0 ? NQL * V * B3 : 1];  // lQi^k slices t < NQL, [t][var][node]
   __shared__ T sQ[USE_NCP ? V * B3 : 1];
-  __shared__ T sK[B2];   // Kxi[n][l]
-  __shared__ T sDu[B2];  // dudx[l][n]
-  __shared__ T sW[B];    // Gauss-Legendre weights
+  __shared__ T sDu[USE_NCP ? B2 : 1];  // dudx[l][n]
   __shared__ T sRed[2 * (NT / kWave)];
 
   T* const out_lduh = static_cast<T*>(a.lduh);
@@ -173,11 +169,9 @@ __global__ __launch_bounds__(node_threads(B), (predictor_min_waves<B, TERMS, T>(
     return;
   }
 
-  for (int i = tid; i < B2; i += NT) {
-    sK[i] = tc<T>(exa_kxi[N][i / B][i % B]);
-    sDu[i] = tc<T>(exa_dudx[N][i / B][i % B]);
+  if constexpr (USE_NCP) {
+    for (int i = tid; i < B2; i += NT) sDu[i] = tc<T>(exa_dudx[N][i / B][i % B]);
   }
-  for (int i = tid; i < B; i += NT) sW[i] = tc<T>(exa_gl_weights[N][i]);
 
   const int patch = a.cell_patch ? a.cell_patch[cell] : 0;
   const double* dxp = a.cell_patch ? a.dx + (size_t)patch * 3 : a.dx + cell * a.dx_stride;
@@ -225,10 +219,10 @@ __global__ __launch_bounds__(node_threads(B), (predictor_min_waves<B, TERMS, T>(
       qi_set(t, m, q0[m]);
   T qn[B][V];
   int iters = MAX_ITER;
-  // Float form of a flux-only PDE: the first Picard iteration in closed form
-  // and the time-averaged fluxes accumulated while the iterations run (see
-  // below); the double form keeps the reference's order of operations.
-  constexpr bool FLOAT_FLUX_ONLY = !IS_FP64 && USE_FLUX && !USE_SRC_NCP;
+  // The first Picard iteration in closed form (see below); a call that exports
+  // the temporaries evaluates every slice of it.
+  constexpr bool FIRST_CLOSED = !EXPORT;
+  constexpr bool FLOAT_FLUX_ONLY = !IS_FP64 && USE_FLUX && !USE_SRC_NCP;  // see ACC_FH
   // accumulating the averages needs 3V more registers: only at B = 5, 6 and
   // 8, where they fit the wavefronts per SIMD that LDS allows (B = 6 and 8
   // with the register cap of predictor_min_waves: 124 and 166 registers; the
@@ -247,26 +241,24 @@ __global__ __launch_bounds__(node_threads(B), (predictor_min_waves<B, TERMS, T>(
   // their occupancy).
   constexpr bool ACC_SH = USE_SRC_NCP && !USE_FLUX;
   T sh[V];
-  const T iweight = T(1.0) / w3;
   __syncthreads();
 
-  // Float form: the quadrature weights and dt/dx of the line contraction are
-  // applied per node in phase 3 instead of per line value in phase 2:
-  // us_d / w^3 = w_t dt / (dx_d w_d), w_d the node's weight along d.
-  const T g_node[3] = {dt * invDx[0] / wx, dt * invDx[1] / wy, dt * invDx[2] / wz};
+  const T gd[3] = {dt * invDx[0], dt * invDx[1], dt * invDx[2]};
   // Phase 2 tasks per direction: one (variable m, line) each, NTD of them in
   // RD rounds over the workgroup.
   constexpr int NTD = B2 * V;
   constexpr int RD = (NTD + NT - 1) / NT;
 
-  // Phase 2 of a time slice (line owners): per direction d, one task = one
-  // (variable, line); out(l) = sum_n (us * F(n)) * Kxi[n][l] along the line,
-  // with us = w_t w_a w_b dt / dx_d (:152-236) -- in the float form us is
-  // applied per node in phase 3 instead.  Directions run one after the other
-  // with compile-time strides; Kxi comes in as constants.  A task reads its
-  // whole line before writing the results back to the same positions, and no
-  // other task touches them: the contraction is in place.  Ends with a barrier.
-  auto contract_lines = [&](const T wt) __device__ __attribute__((always_inline)) {
+  // Line contractions by the line owners, in place: per direction d, one task =
+  // one (variable, line).  A task reads its whole line before writing the
+  // results back to the same positions, and no other task touches them.
+  // Directions run one after the other with compile-time strides; the
+  // operator's entries come in as constants.  VOLUME: sum_n Kxi[l][n] F(n) of
+  // the volume integral; otherwise the derivative at every node (phase 2 of a
+  // time slice, :152-236: the reference's Kxi with the weight w_l of the result
+  // taken out, so that phase 3 needs one factor w_t dt / dx_d per slice).
+  // Ends with a barrier.
+  auto contract_lines = [&]<bool VOLUME>() __device__ __attribute__((always_inline)) {
 #pragma unroll
     for (int r = 0; r < RD; ++r) {
       if (tid + r * NT < NTD) {
@@ -274,29 +266,18 @@ __global__ __launch_bounds__(node_threads(B), (predictor_min_waves<B, TERMS, T>(
         const int m = task / B2, line = task - (task / B2) * B2;
         const int la = line / B, lb = line - (line / B) * B;
         // line starts: x-lines (z,y) stride 1, y-lines (z,x) stride B,
-        // z-lines (y,x) stride B^2; the weights are w_la, w_lb
+        // z-lines (y,x) stride B^2
         const int off0 = m * B3 + line * B, off1 = m * B3 + la * B2 + lb, off2 = m * B3 + line;
-        const T wa = sW[la], wb = sW[lb];
 #pragma unroll
         for (int d = 0; d < 3; ++d) {
           const int stride = d == 0 ? 1 : (d == 1 ? B : B2);
           const int o = d * V * B3 + (d == 0 ? off0 : (d == 1 ? off1 : off2));
-          T f[B];
-          if constexpr (IS_FP64) {
-            const T us = wt * wa * wb * dt * invDx[d];
+          T f[B], out[B];
 #pragma unroll
-            for (int n = 0; n < B; ++n) f[n] = us * sF[o + n * stride];
-          } else {
+          for (int n = 0; n < B; ++n) f[n] = sF[o + n * stride];
+          contract_halves<B, VOLUME>(f, out);
 #pragma unroll
-            for (int n = 0; n < B; ++n) f[n] = sF[o + n * stride];
-          }
-#pragma unroll
-          for (int l = 0; l < B; ++l) {
-            T acc = T(0);
-#pragma unroll
-            for (int n = 0; n < B; ++n) acc += f[n] * tc<T>(exa_kxi[N][n][l]);
-            sF[o + l * stride] = acc;
-          }
+          for (int l = 0; l < B; ++l) sF[o + l * stride] = out[l];
         }
       }
     }
@@ -305,11 +286,9 @@ __global__ __launch_bounds__(node_threads(B), (predictor_min_waves<B, TERMS, T>(
 
 #pragma unroll 1
   for (int iter = 0; iter < MAX_ITER; ++iter) {
-    // rhs0 = w^3 FLCoeff[t] luh is loop invariant; keeping B*V copies of it live
-    // across iterations costs more registers than recomputing it per slice.
-    T w3i = w3;
-    asm volatile("" : "+v"(w3i));
-    T q0i[V];  // the same for the float form's FLCoeff[t] luh
+    // FLCoeff[t] luh is loop invariant; keeping B V copies of it live across
+    // iterations costs more registers than recomputing it per slice.
+    T q0i[V];
 #pragma unroll
     for (int m = 0; m < V; ++m) {
       q0i[m] = q0[m];
@@ -343,13 +322,6 @@ __global__ __launch_bounds__(node_threads(B), (predictor_min_waves<B, TERMS, T>(
       for (int m = 0; m < V; ++m) Q[m] = qi(t, m);
 #pragma unroll
       for (int m = V; m < D; ++m) Q[m] = q0[m];
-      // Float form, first iteration: every slice of the initial iterate equals
-      // luh, and phase 2 does not depend on t there, so the fluxes and line
-      // contractions of slice 0 (still in LDS) serve every slice (the same
-      // inputs give the same values).  The double form keeps w_t inside the
-      // contraction, as the reference, and evaluates every slice.
-      const bool reuse = !IS_FP64 && iter == 0 && t > 0;
-      if (!reuse) {
       // phase 1 (node owners): fluxes of this time slice -> sF[dir][var][node]
       if (USE_FLUX) {
         T F[3][V];
@@ -381,61 +353,31 @@ __global__ __launch_bounds__(node_threads(B), (predictor_min_waves<B, TERMS, T>(
       }
       __syncthreads();
 
-      if (USE_FLUX) contract_lines(wt);
-      }  // !reuse
+      if (USE_FLUX) contract_lines.template operator()<false>();
 
-      // phase 3 (node owners): rhs = w^3 FLCoeff[t] luh - contributions (+ S dt w^4)
-      // (:124-141, :238-276); lQi_new(l) += iweight * rhs * iK1[l][t] (:292-299, n = t)
+      // phase 3 (node owners): rhs / w^3 = FLCoeff[t] luh - sum_d w_t dt / dx_d
+      // dF_d (+ S w_t dt) (:124-141, :238-276); lQi_new(l) += rhs / w^3
+      // iK1[l][t] (:292-299, n = t)
       const T fl_t = tc<T>(exa_fl_coeff[N][t]);
-      if constexpr (!IS_FP64) {
-        // float form: ir = rhs / w^3 directly, weights folded per node
-        T ir[V];
-        const T wg[3] = {wt * g_node[0], wt * g_node[1], wt * g_node[2]};
-#pragma unroll
-        for (int m = 0; m < V; ++m) {
-          ir[m] = fl_t * q0i[m];
-          if (USE_FLUX) {
-            ir[m] -= wg[0] * sF[(0 * V + m) * B3 + node];
-            ir[m] -= wg[1] * sF[(1 * V + m) * B3 + node];
-            ir[m] -= wg[2] * sF[(2 * V + m) * B3 + node];
-          }
-        }
-        if (USE_SRC_NCP) {
-          T S[V];
-          source_ncp<B, PDE, USE_SOURCE, USE_NCP>(Q, sQ, sDu, invDx, z, y, x, S);
-          const T us = wt * dt;
-#pragma unroll
-          for (int m = 0; m < V; ++m) ir[m] += us * S[m];
-          if constexpr (ACC_SH) {
-            // time average of the slice sources of this iterate (:367-396)
-#pragma unroll
-            for (int m = 0; m < V; ++m) sh[m] += S[m] * wt;
-          }
-        }
-#pragma unroll
-        for (int m = 0; m < V; ++m)
-#pragma unroll
-          for (int l = 0; l < B; ++l) qn[l][m] += ir[m] * tc<T>(exa_ik1[N][l][t]);
-        if (USE_FLUX || USE_NCP) __syncthreads();  // the next slice rewrites sF / sQ
-        return;
-      }
-      T r[V];
+      T ir[V];
+      const T wg[3] = {wt * gd[0], wt * gd[1], wt * gd[2]};
 #pragma unroll
       for (int m = 0; m < V; ++m) {
-        r[m] = w3i * fl_t * q0[m];
+        ir[m] = fl_t * q0i[m];
         if (USE_FLUX) {
-          r[m] -= sF[(0 * V + m) * B3 + node];
-          r[m] -= sF[(1 * V + m) * B3 + node];
-          r[m] -= sF[(2 * V + m) * B3 + node];
+          ir[m] -= wg[0] * sF[(0 * V + m) * B3 + node];
+          ir[m] -= wg[1] * sF[(1 * V + m) * B3 + node];
+          ir[m] -= wg[2] * sF[(2 * V + m) * B3 + node];
         }
       }
       if (USE_SRC_NCP) {
         T S[V];
         source_ncp<B, PDE, USE_SOURCE, USE_NCP>(Q, sQ, sDu, invDx, z, y, x, S);
-        const T us = wt * wz * wy * wx * dt;
+        const T us = wt * dt;
 #pragma unroll
-        for (int m = 0; m < V; ++m) r[m] += us * S[m];
+        for (int m = 0; m < V; ++m) ir[m] += us * S[m];
         if constexpr (ACC_SH) {
+          // time average of the slice sources of this iterate (:367-396)
 #pragma unroll
           for (int m = 0; m < V; ++m) sh[m] += S[m] * wt;
         }
@@ -446,59 +388,63 @@ __global__ __launch_bounds__(node_threads(B), (predictor_min_waves<B, TERMS, T>(
         }
       }
 #pragma unroll
-      for (int m = 0; m < V; ++m) {
-        const T ir = iweight * r[m];
+      for (int m = 0; m < V; ++m)
 #pragma unroll
-        for (int l = 0; l < B; ++l) qn[l][m] += ir * tc<T>(exa_ik1[N][l][t]);
-      }
+        for (int l = 0; l < B; ++l) qn[l][m] += ir[m] * tc<T>(exa_ik1[N][l][t]);
       if (USE_FLUX || USE_NCP) __syncthreads();  // the next slice rewrites sF / sQ
     };
-    if (FLOAT_FLUX_ONLY && iter == 0) {
-      // First iteration of the float form: every slice of the initial
-      // iterate equals luh, so the slices share one flux contraction S and
-      // lQi^1(l) = sum_t iK1[l][t] (FLCoeff[t] luh - w_t S)
-      //          = (sum_t iK1[l][t] FLCoeff[t]) luh - (sum_t iK1[l][t] w_t) S,
-      // coefficients formed in double from the tables.
-      T F[3][V];
-      {
-        T Q[D];
+    if (FIRST_CLOSED && iter == 0) {
+      // Every slice of the initial iterate equals luh, so one evaluation
+      // R = sum_d dt / dx_d dF_d - dt S serves all slices:
+      // lQi^1(l) = sum_t iK1[l][t] (FLCoeff[t] luh - w_t R) = a_l luh - b_l R,
+      // a_l and b_l formed in double from the tables: one slice's evaluation
+      // instead of B.  In double at N=5 (64,000 cells, 4 iterations), with the
+      // halved contractions: 6.1 -> 5.1 ms; N=3 1.30 -> 1.07 ms, elastic N=4
+      // 5.6 -> 4.0 ms.
+      T Q[D], R[V];
 #pragma unroll
-        for (int m = 0; m < D; ++m) Q[m] = m < V ? q0i[m < V ? m : 0] : q0[m];
+      for (int m = 0; m < D; ++m) Q[m] = m < V ? q0i[m < V ? m : 0] : q0[m];
+      double sw = 0.0;
+#pragma unroll
+      for (int t = 0; t < B; ++t) sw += exa_gl_weights[N][t];
+      const T sumw = tc<T>(sw);
+      if constexpr (USE_FLUX) {
+        T F[3][V];
         PDE::flux(Q, F);
+#pragma unroll
+        for (int d = 0; d < 3; ++d)
+#pragma unroll
+          for (int m = 0; m < V; ++m) {
+            sF[(d * V + m) * B3 + node] = F[d][m];
+            if constexpr (ACC_FH) fh[d][m] = F[d][m] * sumw;
+          }
       }
-      T sumw = T(0);
-      {
-        double sw = 0.0;
+      if constexpr (USE_NCP) {
 #pragma unroll
-        for (int t = 0; t < B; ++t) sw += exa_gl_weights[N][t];
-        sumw = tc<T>(sw);
+        for (int m = 0; m < V; ++m) sQ[m * B3 + node] = Q[m];
       }
-#pragma unroll
-      for (int d = 0; d < 3; ++d)
-#pragma unroll
-        for (int m = 0; m < V; ++m) {
-          sF[(d * V + m) * B3 + node] = F[d][m];
-          if constexpr (ACC_FH) fh[d][m] = F[d][m] * sumw;
-        }
       __syncthreads();
-      contract_lines(T(0));
-      T S[V];
+      if constexpr (USE_FLUX) contract_lines.template operator()<false>();
 #pragma unroll
       for (int m = 0; m < V; ++m)
-        S[m] = g_node[0] * sF[(0 * V + m) * B3 + node] + g_node[1] * sF[(1 * V + m) * B3 + node] +
-               g_node[2] * sF[(2 * V + m) * B3 + node];
+        R[m] = USE_FLUX ? gd[0] * sF[(0 * V + m) * B3 + node] + gd[1] * sF[(1 * V + m) * B3 + node] +
+                              gd[2] * sF[(2 * V + m) * B3 + node]
+                        : T(0);
+      if constexpr (USE_SRC_NCP) {
+        T S[V];
+        source_ncp<B, PDE, USE_SOURCE, USE_NCP>(Q, sQ, sDu, invDx, z, y, x, S);
 #pragma unroll
-      for (int l = 0; l < B; ++l) {
-        double al = 0.0, bl = 0.0;
-#pragma unroll
-        for (int t = 0; t < B; ++t) {
-          al += exa_ik1[N][l][t] * exa_fl_coeff[N][t];
-          bl += exa_ik1[N][l][t] * exa_gl_weights[N][t];
+        for (int m = 0; m < V; ++m) {
+          R[m] -= dt * S[m];
+          if constexpr (ACC_SH) sh[m] = S[m] * sumw;
         }
-#pragma unroll
-        for (int m = 0; m < V; ++m) qn[l][m] = tc<T>(al) * q0i[m] - tc<T>(bl) * S[m];
       }
-      __syncthreads();  // the next iteration rewrites sF
+#pragma unroll
+      for (int l = 0; l < B; ++l)
+#pragma unroll
+        for (int m = 0; m < V; ++m)
+          qn[l][m] = tc<T>(exa_folded.a[N][l]) * q0i[m] - tc<T>(exa_folded.b[N][l]) * R[m];
+      __syncthreads();  // the next iteration rewrites sF / sQ
     } else if constexpr (SPLIT) {
 #pragma unroll 1
       for (int t = 0; t < NQL; ++t) picard_slice(t);
@@ -685,67 +631,16 @@ __global__ __launch_bounds__(node_threads(B), (predictor_min_waves<B, TERMS, T>(
     T acc[V];
 #pragma unroll
     for (int m = 0; m < V; ++m) acc[m] = T(0);
-    if constexpr (!IS_FP64) {
-      // float form: the directional contractions sum_n Kxi[l][n] lFhi_d(n) as
-      // line tasks in place (as in phase 2), then each node sums its three
-      // directions with their weights
-      if (USE_FLUX) {
-        __syncthreads();  // the extrapolation has read sF
+    if constexpr (USE_FLUX) {
+      // the directional contractions sum_n Kxi[l][n] lFhi_d(n) as line tasks in
+      // place, then each node sums its three directions with their weights
+      __syncthreads();  // the extrapolation has read sF
+      contract_lines.template operator()<true>();
+      const T us[3] = {wz * wy * invDx[0], wz * wx * invDx[1], wy * wx * invDx[2]};
 #pragma unroll
-        for (int r = 0; r < RD; ++r) {
-          if (tid + r * NT < NTD) {
-            const int task = tid + r * NT;
-            const int m = task / B2, line = task - (task / B2) * B2;
-            const int la = line / B, lb = line - (line / B) * B;
-#pragma unroll
-            for (int d = 0; d < 3; ++d) {
-              const int stride = d == 0 ? 1 : (d == 1 ? B : B2);
-              const int o = (d * V + m) * B3 + (d == 0 ? line * B : (d == 1 ? la * B2 + lb : line));
-              T f[B];
-#pragma unroll
-              for (int n = 0; n < B; ++n) f[n] = sF[o + n * stride];
-#pragma unroll
-              for (int l = 0; l < B; ++l) {
-                T c = T(0);
-#pragma unroll
-                for (int n = 0; n < B; ++n) c += f[n] * tc<T>(exa_kxi[N][l][n]);
-                sF[o + l * stride] = c;
-              }
-            }
-          }
-        }
-        __syncthreads();
-        const T us[3] = {wz * wy * invDx[0], wz * wx * invDx[1], wy * wx * invDx[2]};
-#pragma unroll
-        for (int m = 0; m < V; ++m)
-          acc[m] = us[0] * sF[(0 * V + m) * B3 + node] + us[1] * sF[(1 * V + m) * B3 + node] +
-                   us[2] * sF[(2 * V + m) * B3 + node];
-      }
-    } else if (USE_FLUX) {
-      {
-        const T us = wz * wy * invDx[0];
-        const T* row = sF + (0 * V) * B3 + (z * B + y) * B;
-#pragma unroll
-        for (int m = 0; m < V; ++m)
-#pragma unroll
-          for (int n = 0; n < B; ++n) acc[m] += sK[x * B + n] * row[m * B3 + n] * us;
-      }
-      {
-        const T us = wz * wx * invDx[1];
-        const T* col = sF + (1 * V) * B3 + z * B2 + x;
-#pragma unroll
-        for (int m = 0; m < V; ++m)
-#pragma unroll
-          for (int n = 0; n < B; ++n) acc[m] += sK[y * B + n] * col[m * B3 + n * B] * us;
-      }
-      {
-        const T us = wy * wx * invDx[2];
-        const T* col = sF + (2 * V) * B3 + y * B + x;
-#pragma unroll
-        for (int m = 0; m < V; ++m)
-#pragma unroll
-          for (int n = 0; n < B; ++n) acc[m] += sK[z * B + n] * col[m * B3 + n * B2] * us;
-      }
+      for (int m = 0; m < V; ++m)
+        acc[m] = us[0] * sF[(0 * V + m) * B3 + node] + us[1] * sF[(1 * V + m) * B3 + node] +
+                 us[2] * sF[(2 * V + m) * B3 + node];
     }
     if (USE_SRC_NCP) {
 #pragma unroll

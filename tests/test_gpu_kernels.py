@@ -97,6 +97,46 @@ def test_batch_predictor_volume_vs_oracle(exa, oracle, order):
         assert rel_max(r["lduh"][c * nb3:(c + 1) * nb3], lduh) < TOL, c
 
 
+@pytest.mark.parametrize("pde,order", [("euler", n) for n in range(2, 8)] + [("elastic", n) for n in range(2, 6)])
+def test_batch_predictor_first_iteration_vs_oracle(exa, oracle, pde, order):
+    """Cells that leave the Picard loop after its first iteration, whose slices
+    share one evaluation, beside cells that do not: the same counts and, since
+    the shared evaluation is the same linear map summed in another order, the
+    same results to TOL."""
+    rng = np.random.default_rng(7 + order)
+    n, B = 6, order + 1
+    if pde == "euler":
+        s, es = oracle.make_solver(order, 5, 0), exa.euler_solver(order)
+        luh = smooth_euler_cells(rng, n, order).reshape(n, -1)
+        luh[: n // 2] = np.tile(luh[: n // 2, :5], B ** 3)  # uniform: nothing changes
+    else:
+        s, es = oracle.elastic_solver(order), exa.elastic_solver(order)
+        x = np.linspace(0.0, 1.0, B ** 3)[None, :, None]
+        q = rng.uniform(-1, 1, (n, 1, 9)) * np.sin(x + np.arange(9))
+        q[: n // 2] = q[: n // 2, :1]
+        luh = np.concatenate([q, np.broadcast_to([2.0, 1.0, 2.5], (n, B ** 3, 3))], -1).reshape(n, -1)
+    D, V = es.D, es.num_variables
+    dx = np.tile([0.05, 0.04, 0.06], (n, 1))
+    dt = 0.5 * min(oracle.stable_dt(s, luh[c], dx[c]) for c in range(n))
+    print(f"case: batch predictor, first iteration, {pde} N={order}", flush=True)
+    r = exa.batch_predictor_volume(es, luh.ravel(), dx, dt)
+    its = []
+    for c in range(n):
+        o = oracle.space_time_predictor(s, luh[c], dx[c], dt)
+        its.append(o["iters"])
+        assert r["iters"][c] == o["iters"], c
+        for k, size in (("lQhbnd", 6 * B * B * D), ("lFhbnd", 6 * B * B * V)):
+            assert np.abs(r[k][c * size:(c + 1) * size] - o[k]).max() <= TOL * np.abs(luh[c]).max(), (c, k)
+        lduh = oracle.volume_integral(s, o["lFhi"], dx[c])
+        # For a uniform state the exact result is 0: the terms of a derivative cancel.  Each is at
+        # most (operator entry) x (flux, or for the elastic product coefficient x state) / dx, so the
+        # rounding bound is eps times that; coefficients here are at most lambda + 2 mu = 4.
+        term = max(np.abs(o["lFhi"]).max(), 4.0 * np.abs(luh[c]).max())
+        scale = max(np.abs(lduh).max(), term / dx[c].min())
+        assert np.abs(r["lduh"][c * B ** 3 * V:(c + 1) * B ** 3 * V] - lduh).max() <= TOL * scale, c
+    assert min(its) == 1 and max(its) > 1
+
+
 def test_golden_volume_integral(exa):
     """testVolumeIntegralNonlinear::lduh (GenericEulerKernelTest3D.cpp:204-215
     inputs, dx = 0.05: the mesh size the golden data was made with)."""
