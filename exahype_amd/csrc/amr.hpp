@@ -11,14 +11,14 @@ constexpr int kAmrMaxLevelDelta = 6;  // 3^6 = 729 subintervals per direction
 // A batch of transfers between blocks of B^NDIM nodes x nv values (volumes:
 // (z,y,x,var); faces: (b,a,var)).  items: 5 ints per transfer (destination
 // block, source block, subinterval index per direction in [0, 3^level_delta);
-// faces use the first two).  Prolongation: one workgroup per item, the
+// faces use the first two).  Prolongation: one wavefront per item, the
 // destination overwritten.  Restriction: one workgroup per destination k over
 // items [ptr[k], ptr[k+1]), which must share one destination block; their
 // restricted blocks are added to it in list order.  Items with an index out of
 // range (or a mismatched destination) are skipped and set *error.  Every
 // destination block may appear once per launch (one item of a prolongation,
-// one range of a restriction): each workgroup claims its destination's bit in
-// `claimed` (dst_blocks bits, zero on entry) before it writes, and a workgroup
+// one range of a restriction): each transfer (or range) claims its destination's
+// bit in `claimed` (dst_blocks bits, zero on entry) before it writes, and one
 // that finds the bit taken writes nothing and sets *error.
 struct AmrArgs {
   double* dst;

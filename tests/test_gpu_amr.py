@@ -197,3 +197,35 @@ def test_batch_rejects_repeated_destinations(exa, oracle):
     ok_items = exa.DeviceArray(np.array([(0, 0, 0, 0, 0), (0, 1, 1, 0, 0), (1, 2, 2, 2, 2)], dtype=np.int32))
     ok_ptr = exa.DeviceArray(np.array([0, 2, 3], dtype=np.int32))
     exa.volume_restriction_batch(s, exa.DeviceArray(start), d_fin, ok_ptr, ok_items, 1)
+
+
+@pytest.mark.parametrize("order,nv,children", [(1, 5, (1, 3, 0, 27)), (2, 5, (4, 5, 1, 0)), (3, 5, (27, 2, 8, 9)),
+                                               (4, 12, (5, 0, 4, 3)), (5, 5, (27, 1, 6, 0)), (5, 12, (3, 5, 0, 1))])
+def test_batches_uneven_ranges_vs_oracle(exa, oracle, order, nv, children):
+    """Both directions with 5 values per node and another count, destinations
+    with no, few and many transfers (a destination's transfers run four at a
+    time), a number of transfers that fills no whole workgroup."""
+    print(f"case: AMR batches N={order} nv={nv} children={children}", flush=True)
+    rng = np.random.default_rng(order * 100 + nv)
+    s, os_ = (_solvers(exa, oracle, order, npar=0) if nv == 5 else
+              (exa.elastic_solver(order), oracle.elastic_solver(order)))
+    blk = (order + 1) ** 3 * nv
+    nfine = sum(children)
+    sub = rng.integers(0, 3, (nfine, 3))
+    owner = np.repeat(np.arange(len(children)), children)
+    order_ = rng.permutation(nfine)  # fine blocks in any order
+    items = np.column_stack([order_, owner, sub]).astype(np.int32)
+    ptr = np.concatenate([[0], np.cumsum(children)]).astype(np.int32)
+    coarse = rng.standard_normal((len(children), blk))
+    d_fine = exa.DeviceArray(np.zeros((nfine, blk)))
+    exa.volume_prolongation_batch(s, d_fine, exa.DeviceArray(coarse), exa.DeviceArray(items), 1)
+    fine = d_fine.get()
+    for it in items:
+        assert _rel(fine[it[0]], oracle.volume_unknowns_prolongation(os_, coarse[it[1]], 0, 1, it[2:])) <= 1e-12
+    acc, d_acc = coarse.copy(), exa.DeviceArray(coarse)
+    fine_in = rng.standard_normal((nfine, blk))
+    exa.volume_restriction_batch(s, d_acc, exa.DeviceArray(fine_in), exa.DeviceArray(ptr),
+                                 exa.DeviceArray(np.ascontiguousarray(items[:, [1, 0, 2, 3, 4]])), 1)
+    for it in items:
+        acc[it[1]] = oracle.volume_unknowns_restriction(os_, acc[it[1]], fine_in[it[0]], 0, 1, it[2:])
+    assert _rel(d_acc.get(), acc) <= 1e-12
