@@ -792,17 +792,17 @@ def cpu_baseline_elastic(seconds, threads=16):
 
 def linear_roofline(stages, n, B):
     """Roofline of the linear predictor (the linear form's dominant kernel): it
-    reads luh (B^3 x 12 doubles) and writes lduh (B^3 x 9) and both face arrays
-    (6 B^2 x (12 + 9)) per cell; launch time from the grid's HIP events."""
+    reads luh (B^3 x 12 doubles) and writes lduh (B^3 x 9) and the face states
+    (6 B^2 x 12) per cell; launch time from the grid's HIP events."""
     ms, launches = stages["predictor"]
     avg = ms / max(launches, 1)
-    alg = n ** 3 * (B ** 3 * 12 + B ** 3 * 9 + 6 * B * B * 21) * 8
+    alg = n ** 3 * (B ** 3 * 12 + B ** 3 * 9 + 6 * B * B * 12) * 8
     achieved = alg / (avg * 1e-3) / 1e9
     return dict(bound="hbm", achieved=round(achieved, 1), peak=HBM_PEAK_GBS, unit="GB/s",
                 frac=round(achieved / HBM_PEAK_GBS, 4), traffic=linear_predictor_traffic(),
-                kernel="linear_predictor_kernel<5, Elastic> (Cauchy-Kowalevski + linear volume integral)",
+                kernel="linear_grid_predictor_kernel<5, Elastic> (Cauchy-Kowalevski + linear volume integral)",
                 avg_launch_ms=round(avg, 4), algorithmic_bytes_per_launch=alg,
-                note="latency-bound on LDS (neither HBM nor ALU saturated)")
+                note="LDS-bound: the gradients read every line entry from LDS")
 
 
 def elastic_roofline(r, B, peak, valu_peak, kernel):

@@ -431,20 +431,6 @@ hipError_t launch_update(const SolverDesc& sd, int mode, const UpdateArgs& a, lo
   if (ncells <= 0) return hipSuccess;
   return dispatch_pde(sd, [&]<int B, class PDE>() -> hipError_t {
     const dim3 grid((unsigned)ncells), block(node_threads(B));
-    if (sd.linear && (mode & kUpdSurface)) {  // the linear solvers' surface integral
-      if constexpr (std::is_same_v<PDE, Elastic> || std::is_same_v<PDE, Euler<1>>) {
-        if (sd.precision != kFP64) return hipErrorNotSupported;
-        if (mode == (kUpdSurface | kUpdUpdate))
-          hipLaunchKernelGGL((update_kernel<B, PDE, true, true, false, double, true>), grid, block, 0, s, a);
-        else if (mode == (kUpdSurface | kUpdWriteLduh))
-          hipLaunchKernelGGL((update_kernel<B, PDE, true, false, true, double, true>), grid, block, 0, s, a);
-        else
-          return hipErrorInvalidValue;
-        return hipGetLastError();
-      } else {
-        return hipErrorNotSupported;
-      }
-    }
     if (sd.precision == kFP32Bulk) {
       if (mode == (kUpdSurface | kUpdUpdate))
         hipLaunchKernelGGL((update_kernel<B, PDE, true, true, false, float>), grid, block, 0, s, a);

@@ -513,14 +513,13 @@ hipError_t launch_predict(exa_grid* g, const double* dt, const int* run_if = nul
     la.luh = g->luh;
     la.lduh = static_cast<double*>(g->lduh);
     la.lQhbnd = static_cast<double*>(g->lQhbnd);
-    la.lFhbnd = static_cast<double*>(g->lFhbnd);
     la.dx = g->d_dx;
     la.dx_stride = 0;
     la.dt = dt;
     la.cell0 = 0;
     if (run_if) return hipErrorNotSupported;  // fused time stepping is for nonlinear solvers
     return staged(g, EXA_STAGE_PREDICTOR,
-                  [&] { return exa::launch_linear_predictor(g->sd, false, la, g->ncells, g->stream); });
+                  [&] { return exa::launch_linear_grid_predictor(g->sd, la, g->ncells, g->stream); });
   }
   exa::PredictorArgs a{};
   a.luh = g->luh;
@@ -547,7 +546,7 @@ hipError_t launch_predict(exa_grid* g, const double* dt, const int* run_if = nul
 // The corrector of one step: Riemann problems, surface integral, update with
 // the corrector dt, the admissible dt of every cell into the dt slots.
 hipError_t launch_correct(exa_grid* g) {
-  if (!g->sd.linear && (g->fused_corrector || g->user)) {
+  if (g->sd.linear || g->fused_corrector || g->user) {
     exa::CorrectorArgs ca{};
     ca.luh = g->luh;
     ca.lduh = g->lduh;
@@ -573,9 +572,7 @@ hipError_t launch_correct(exa_grid* g) {
     });
   }
   exa::RiemannArgs ra{g->faces, g->nfaces, g->lQhbnd, g->lFhbnd};
-  hipError_t e = staged(g, EXA_STAGE_RIEMANN, [&] {
-    return g->sd.linear ? exa::launch_linear_riemann(g->sd, ra, g->stream) : exa::launch_riemann(g->sd, ra, g->stream);
-  });
+  hipError_t e = staged(g, EXA_STAGE_RIEMANN, [&] { return exa::launch_riemann(g->sd, ra, g->stream); });
   if (e != hipSuccess) return e;
   exa::UpdateArgs ua{};
   ua.luh = g->luh;
@@ -623,10 +620,6 @@ hipError_t launch_one_step(exa_grid* g) {
 static int grid_create_impl(const SolverDesc& sd, const exa_user_solver* user, int nx, int ny, int nz,
                             const double* lo, const double* hi, int boundary, exa_grid** out) {
   const bool periodic = boundary == EXA_BC_PERIODIC;
-  // Linear solvers with transmissive boundaries: the linear Riemann solver's
-  // fluctuations vanish at a boundary face (outside = inside), so those faces
-  // join the face list to be zeroed.
-  const bool linear_bc = sd.linear && !periodic;
   if ((double)nx * ny * nz > 2.0e9) return EXA_E_INVALID;
   exa_grid* g = new exa_grid();
   g->sd = sd;
@@ -654,7 +647,8 @@ static int grid_create_impl(const SolverDesc& sd, const exa_user_solver* user, i
   A((void**)&g->luh, sizeof(double) * g->ncells * z.B3 * z.D);
   A((void**)&g->lduh, g->bulk * g->ncells * z.B3 * z.V);
   A((void**)&g->lQhbnd, g->bulk * g->ncells * 6 * z.B2 * z.D);
-  A((void**)&g->lFhbnd, g->bulk * g->ncells * 6 * z.B2 * z.V);
+  // a linear grid's corrector takes the states only and needs no face list
+  if (!sd.linear) A((void**)&g->lFhbnd, g->bulk * g->ncells * 6 * z.B2 * z.V);
   A((void**)&g->d_dx, sizeof(double) * 3);
   A((void**)&g->iters, sizeof(int) * g->ncells);
   if (const size_t wsb = sd.linear ? 0 : exa::predictor_ws_bytes_per_cell(sd)) {
@@ -667,9 +661,10 @@ static int grid_create_impl(const SolverDesc& sd, const exa_user_solver* user, i
   // against boundaryValues' outside state (ADERDGSolver.cpp:2893-2966), and
   // with transmissive values (outside = inside) Rusanov returns the inner
   // flux unchanged, so those faces need no work.
-  g->nfaces = periodic ? 3 * g->ncells : (long)(nx - 1) * ny * nz + (long)nx * (ny - 1) * nz + (long)nx * ny * (nz - 1);
-  if (linear_bc) g->nfaces += 2 * ((long)ny * nz + (long)nx * nz + (long)nx * ny);
-  A((void**)&g->faces, sizeof(FaceDesc) * g->nfaces);
+  g->nfaces = sd.linear ? 0
+              : periodic ? 3 * g->ncells
+                         : (long)(nx - 1) * ny * nz + (long)nx * (ny - 1) * nz + (long)nx * ny * (nz - 1);
+  if (g->nfaces > 0) A((void**)&g->faces, sizeof(FaceDesc) * g->nfaces);
   A((void**)&g->st, sizeof(exa::StepState));
   g->dt_hist_len = 1 << 16;
   A((void**)&g->dt_hist, sizeof(double) * g->dt_hist_len);
@@ -685,7 +680,7 @@ static int grid_create_impl(const SolverDesc& sd, const exa_user_solver* user, i
     return (int)(((long)k * ny + j) * nx + i);
   };
   long f = 0;
-  for (int dir = 0; dir < 3; ++dir)
+  for (int dir = 0; dir < 3 && g->nfaces > 0; ++dir)
     for (int k = 0; k < nz; ++k)
       for (int j = 0; j < ny; ++j)
         for (int i = 0; i < nx; ++i) {
@@ -696,17 +691,6 @@ static int grid_create_impl(const SolverDesc& sd, const exa_user_solver* user, i
           const int r = dir == 0 ? cid(i + 1, j, k) : (dir == 1 ? cid(i, j + 1, k) : cid(i, j, k + 1));
           faces[f++] = FaceDesc{c, r, dir, 0};
         }
-  if (linear_bc)
-    for (int dir = 0; dir < 3; ++dir)
-      for (int k = 0; k < nz; ++k)
-        for (int j = 0; j < ny; ++j)
-          for (int i = 0; i < nx; ++i) {
-            const int pos = dir == 0 ? i : (dir == 1 ? j : k);
-            const int nmax = dir == 0 ? nx : (dir == 1 ? ny : nz);
-            const int c = cid(i, j, k);
-            if (pos == 0) faces[f++] = FaceDesc{c, c, dir, 1};
-            if (pos == nmax - 1) faces[f++] = FaceDesc{c, c, dir, 2};
-          }
   exa::StepState st0{};
   st0.dt = 0.0;
   st0.t = 0.0;
@@ -714,7 +698,7 @@ static int grid_create_impl(const SolverDesc& sd, const exa_user_solver* user, i
   st0.dt_hist = g->dt_hist;
   st0.dt_hist_len = g->dt_hist_len;
   for (int i = 0; i < exa::kDtSlots; ++i) st0.dt_slots[i] = exa::kDtSlotEmpty;
-  e = hipMemcpy(g->faces, faces.data(), sizeof(FaceDesc) * g->nfaces, hipMemcpyHostToDevice);
+  if (g->nfaces > 0) e = hipMemcpy(g->faces, faces.data(), sizeof(FaceDesc) * g->nfaces, hipMemcpyHostToDevice);
   if (e == hipSuccess) e = hipMemcpy(g->st, &st0, sizeof(st0), hipMemcpyHostToDevice);
   if (e == hipSuccess) e = hipMemcpy(g->d_dx, g->dx, sizeof(double) * 3, hipMemcpyHostToDevice);
   if (e == hipSuccess) e = hipMemset(g->lduh, 0, g->bulk * g->ncells * z.B3 * z.V);

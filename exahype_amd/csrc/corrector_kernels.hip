@@ -34,9 +34,34 @@ static hipError_t launch_corrector_t(const SolverDesc& sd, const CorrectorArgs& 
   return hipGetLastError();
 }
 
+// The linear solvers (elasticity at orders 2..5, the five-variable test solver
+// with one parameter at order 3), FP64.
+template <int B, class PDE>
+static hipError_t launch_linear_corrector_t(const CorrectorArgs& a, hipStream_t s) {
+  if (a.boundary == kBoundaryUser || a.adjust) return hipErrorNotSupported;
+  const long ncells = (long)a.nx * a.ny * a.nz;
+  const long per = (ncells + 7) / 8;
+  hipLaunchKernelGGL((corrector_kernel<B, PDE, false, double, true>), dim3((unsigned)(8 * per)), dim3(node_threads(B)),
+                     0, s, a);
+  return hipGetLastError();
+}
+
+static hipError_t launch_linear_corrector(const SolverDesc& sd, const CorrectorArgs& a, hipStream_t s) {
+  if (sd.precision != kFP64) return hipErrorNotSupported;
+  if (sd.pde == kPdeEuler && sd.npar == 1 && sd.order == 3) return launch_linear_corrector_t<4, Euler<1>>(a, s);
+  if (sd.pde != kPdeElastic) return hipErrorNotSupported;
+  switch (sd.order) {
+    case 2: return launch_linear_corrector_t<3, Elastic>(a, s);
+    case 3: return launch_linear_corrector_t<4, Elastic>(a, s);
+    case 4: return launch_linear_corrector_t<5, Elastic>(a, s);
+    case 5: return launch_linear_corrector_t<6, Elastic>(a, s);
+    default: return hipErrorNotSupported;
+  }
+}
+
 hipError_t launch_corrector(const SolverDesc& sd, const CorrectorArgs& a, hipStream_t s) {
-  if (sd.linear) return hipErrorNotSupported;
   if ((long)a.nx * a.ny * a.nz <= 0) return hipSuccess;
+  if (sd.linear) return launch_linear_corrector(sd, a, s);
   if (sd.pde == kPdeEuler && sd.npar == 0) {
     switch (sd.order) {
       case 2: return launch_corrector_t<3, Euler<0>>(sd, a, s);

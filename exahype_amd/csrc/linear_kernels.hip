@@ -2,8 +2,8 @@
 //
 // Reference semantics followed (K = ExaHyPE/kernels/aderdg/generic/c/3d):
 //   linear_predictor_kernel  K/spaceTimePredictorLinear.cpph:34-443 (Cauchy-Kowalevski
-//                            procedure, time averages, extrapolation)
-//                            + K/volumeIntegralLinear.cpph:21-53 (fused epilogue)
+//                            procedure, time averages, extrapolation), single-cell API
+//   linear_grid_predictor_kernel  a grid's cells: lQhbnd and K/volumeIntegralLinear.cpph:21-53
 //   linear_riemann_kernel    K/riemannSolverLinear.cpph:23-132
 //   linear_volume_kernel     K/volumeIntegralLinear.cpph:21-53
 //   linear_surface_kernel    K/surfaceIntegralLinear.cpph:21-90
@@ -204,18 +204,6 @@ __global__ __launch_bounds__(linear_predictor_threads(B)) void linear_predictor_
     for (size_t e = threadIdx.x; e < (size_t)B4 * V; e += NT3) a.lFi[(size_t)B4 * 3 * V + e] = 0.0;
   }
   __syncthreads();  // lQhi in sQ, lFhi_d in sF[d]
-  if (grp == 0 && active && a.lduh) {  // volumeIntegralLinear, lduh = -w^3 sum_d lFhi_d
-    const double w = exa_gl_weights[N][z] * exa_gl_weights[N][y] * exa_gl_weights[N][x];
-    double* du = a.lduh + cell * (size_t)(B3 * V) + node * V;
-#pragma unroll
-    for (int m = 0; m < V; ++m) {
-      double v = 0.0;
-      v -= w * sF[0][m * B3 + node];
-      v -= w * sF[1][m * B3 + node];
-      v -= w * sF[2][m * B3 + node];
-      du[m] = v;
-    }
-  }
   // Extrapolation to the six faces, :312-436: lQhi (D values) onto every face,
   // lFhi_d onto faces 2d and 2d+1; one thread per face node, all variables.
   for (int e = threadIdx.x; e < 6 * B2; e += NT3) {
@@ -247,6 +235,123 @@ __global__ __launch_bounds__(linear_predictor_threads(B)) void linear_predictor_
   }
 }
 
+// The predictor of a grid's cells.  What the time step needs of the space-time
+// expansion is the time-averaged state (extrapolated to the faces) and the
+// volume integral -w^3 sum_d lFhi_d; with q_{i+1} = -sum_d B_d grad_d q_i the sum
+// of the time-averaged products is that of -q_{i+1}, so one thread per node
+// keeps two averages instead of four, all three directions' products stay in
+// its registers and only q_i goes through LDS.  Against the three direction
+// groups above (their products meeting in LDS, lFhbnd extrapolated and written
+// for nobody): elastic N=4, 68,265 cells, 2.34 -> 0.86 ms.
+template <int B, class PDE>
+__global__ __launch_bounds__(node_threads(B), 4) void linear_grid_predictor_kernel(LinearPredictorArgs a) {
+  constexpr int V = PDE::V, P = PDE::P, D = V + P;
+  constexpr int N = B - 1, B2 = B * B, B3 = B2 * B, NT = node_threads(B);
+  __shared__ double sQ[D * B3];  // q_i [var][node] (rows V.. the parameters); lQhi at the end
+  __shared__ double sDu[B2];     // dudx[l][n]
+  const size_t cell = (size_t)blockIdx.x + a.cell0;
+  const int tid = threadIdx.x;
+  const bool active = tid < B3;
+  const int node = active ? tid : 0;
+  const int z = node / B2, y = (node / B) % B, x = node % B;
+  for (int e = tid; e < B2; e += NT) sDu[e] = exa_dudx[N][e / B][e % B];
+  const double* dxp = a.dx + cell * a.dx_stride;
+  const double rdx[3] = {1.0 / dxp[0], 1.0 / dxp[1], 1.0 / dxp[2]};
+  const double dt = *a.dt;
+  double Q[D];  // only the parameters are held: ncp_dir is linear in the gradient
+  // lQhi = q_0 + sum_{i>0} fac_i q_i, and the products' average sum_i fac_i p_i
+  double qh[V], fh[V];
+  {
+    const double* luh = a.luh + cell * (size_t)(B3 * D) + node * D;
+#pragma unroll
+    for (int m = 0; m < D; ++m) Q[m] = luh[m];
+  }
+#pragma unroll
+  for (int m = 0; m < V; ++m) {
+    qh[m] = Q[m];
+    fh[m] = 0.0;
+  }
+  if (active) {
+#pragma unroll
+    for (int m = 0; m < D; ++m) sQ[m * B3 + node] = Q[m];
+  }
+  double c = 1.0, fac = 0.5 * dt;  // Taylor factors dt^i / (i+1)! of q_i and q_{i+1}, :235-250
+#pragma unroll 1
+  for (int i = 0; i < B; ++i) {
+    __syncthreads();  // q_i complete in sQ
+    double p[V];      // sum_d B_d grad_d q_i (:118-203)
+    auto direction = [&]<int d>() __device__ __attribute__((always_inline)) {
+      constexpr int stride = d == 0 ? 1 : (d == 1 ? B : B2);
+      const int l = d == 0 ? x : (d == 1 ? y : z);
+      const double* const q = sQ + (d == 0 ? (z * B + y) * B : (d == 1 ? z * B2 + x : y * B + x));
+      double w[B], g[V], F[V];
+#pragma unroll
+      for (int n = 0; n < B; ++n) w[n] = sDu[l * B + n];
+#pragma unroll
+      for (int m = 0; m < V; ++m) {
+        double acc = 0.0;
+#pragma unroll
+        for (int n = 0; n < B; ++n) acc += q[m * B3 + n * stride] * w[n];
+        g[m] = rdx[d] * acc;
+        __builtin_amdgcn_sched_barrier(0);  // one line's reads at a time in registers
+      }
+      PDE::template ncp_dir<d>(Q, g, F);
+#pragma unroll
+      for (int m = 0; m < V; ++m) p[m] = d == 0 ? F[m] : p[m] + F[m];
+    };
+    direction.template operator()<0>();
+    direction.template operator()<1>();
+    direction.template operator()<2>();
+    __syncthreads();  // sQ no longer read
+    // q_{i+1} = -p_i (:205-219); the last one is not needed
+#pragma unroll
+    for (int m = 0; m < V; ++m) {
+      fh[m] += c * p[m];
+      if (i + 1 < B) qh[m] -= fac * p[m];
+    }
+    if (active) {
+#pragma unroll
+      for (int m = 0; m < V; ++m) sQ[m * B3 + node] = i + 1 < B ? -p[m] : qh[m];
+    }
+    c = fac;
+    fac *= dt / (i + 3);
+  }
+  __syncthreads();  // lQhi complete in sQ
+  {  // volumeIntegralLinear (K/volumeIntegralLinear.cpph:21-53)
+    const double w = exa_gl_weights[N][z] * exa_gl_weights[N][y] * exa_gl_weights[N][x];
+    double* du = a.lduh + cell * (size_t)(B3 * V) + node * V;
+    if (active) {
+#pragma unroll
+      for (int m = 0; m < V; ++m) du[m] = -w * fh[m];
+    }
+  }
+  // Extrapolation to the six faces (:312-436): one task = (face node, datum k),
+  // k fastest; a task reads its normal line once and forms both faces.
+  double* const qb = a.lQhbnd + cell * (size_t)(6 * B2 * D);
+  auto extrapolate = [&]<int d>() __device__ __attribute__((always_inline)) {
+    constexpr int NTK = B2 * D;
+    constexpr int stride = d == 0 ? 1 : (d == 1 ? B : B2);
+#pragma unroll 2
+    for (int task = tid; task < NTK; task += NT) {
+      const int k = task % D, line = task / D;
+      const int la = line / B, lb = line - (line / B) * B;
+      const double* const q = sQ + k * B3 + (d == 0 ? line * B : (d == 1 ? la * B2 + lb : line));
+      double accL = 0.0, accR = 0.0;
+#pragma unroll
+      for (int l = 0; l < B; ++l) {
+        const double v = q[l * stride];
+        accL += v * exa_fl_coeff[N][l];
+        accR += v * exa_fr_coeff[N][l];
+      }
+      qb[(2 * d) * NTK + task] = accL;
+      qb[(2 * d + 1) * NTK + task] = accR;
+    }
+  };
+  extrapolate.template operator()<0>();
+  extrapolate.template operator()<1>();
+  extrapolate.template operator()<2>();
+}
+
 // One face per wavefront, one face node per lane.  The face averages of both
 // states give the dissipation speed smax and the averaged state Qav; the
 // fluctuations are FL = 0.5 (Bn - smax I)^T (QR - QL) into the left cell's
@@ -271,14 +376,6 @@ __global__ __launch_bounds__(256) void linear_riemann_kernel(RiemannArgs a) {
   const int d = fd.dir;
   double* FL = static_cast<double*>(a.lFhbnd) + ((size_t)fd.left * 6 + 2 * d + 1) * (B2 * V);
   double* FR = static_cast<double*>(a.lFhbnd) + ((size_t)fd.right * 6 + 2 * d) * (B2 * V);
-  if (fd.pad != 0) {
-    // A transmissive boundary face (pad 1: face 2d of cell `right`, pad 2: face
-    // 2d+1 of cell `left`): boundaryValues returns the inside state as the
-    // outside one, so QR - QL = 0 and both fluctuations vanish.
-    double* F = fd.pad == 1 ? FR : FL;
-    for (int e = lane; e < B2 * V; e += kWave) F[e] = 0.0;
-    return;
-  }
   const double* QL = static_cast<const double*>(a.lQhbnd) + ((size_t)fd.left * 6 + 2 * d + 1) * (B2 * D);
   const double* QR = static_cast<const double*>(a.lQhbnd) + ((size_t)fd.right * 6 + 2 * d) * (B2 * D);
   double* const sQL = sStage[w];
@@ -483,6 +580,16 @@ hipError_t launch_linear_predictor(const SolverDesc& sd, bool export_temps, cons
     } else {
       hipLaunchKernelGGL((linear_predictor_kernel<B, PDE, false, false>), grid, block, 0, s, a);
     }
+    return hipGetLastError();
+  });
+}
+
+hipError_t launch_linear_grid_predictor(const SolverDesc& sd, const LinearPredictorArgs& a, long ncells,
+                                        hipStream_t s) {
+  if (ncells <= 0) return hipSuccess;
+  if (!linear_supported(sd) || a.PSi || !a.lduh) return hipErrorNotSupported;
+  return dispatch_linear(sd, [&]<int B, class PDE>() -> hipError_t {
+    hipLaunchKernelGGL((linear_grid_predictor_kernel<B, PDE>), dim3((unsigned)ncells), dim3(node_threads(B)), 0, s, a);
     return hipGetLastError();
   });
 }

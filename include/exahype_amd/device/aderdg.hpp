@@ -33,9 +33,6 @@ struct SolverDesc {
 enum : int { kFP64 = 0, kFP32Bulk = 1 };
 
 // A face between two cells; `left` owns face 2*dir+1, `right` owns face 2*dir.
-// pad: 0 for such a face; in linear grids with transmissive boundaries, 1 marks
-// the boundary face 2*dir of cell `right` and 2 the boundary face 2*dir+1 of
-// cell `left` (the other index is unused).
 struct FaceDesc {
   int left;
   int right;
@@ -164,6 +161,8 @@ struct CorrectorArgs {
   const int* patch_n;
   int slots_per_patch;
 };
+// With sd.linear: the linear Riemann solver and surface integral (periodic or
+// transmissive).
 hipError_t launch_corrector(const SolverDesc& sd, const CorrectorArgs& a, hipStream_t s);
 // Whether the library's instantiation for this solver supports a boundary
 // treatment and the per-step adjustment (the library's PDEs have neither hook).
@@ -249,8 +248,6 @@ hipError_t launch_predictor_mfma(const SolverDesc& sd, const PredictorArgs& a, l
 constexpr long kPredictorWsCells = 4096;
 hipError_t launch_riemann(const SolverDesc& sd, const RiemannArgs& a, hipStream_t s);
 // update_kernel modes: surface integral, solution update, write lduh back.
-// With sd.linear the surface integral is surfaceIntegralLinear (fluctuations,
-// F_{2d+1} FRCoeff + F_{2d} FLCoeff, divided by dx).
 enum : int { kUpdSurface = 1, kUpdUpdate = 2, kUpdWriteLduh = 4 };
 hipError_t launch_update(const SolverDesc& sd, int mode, const UpdateArgs& a, long ncells,
                          hipStream_t s);
@@ -278,9 +275,9 @@ hipError_t launch_euler_ic(const ICArgs& a, hipStream_t s);
 // ---- linear ADER-DG kernels (linear_kernels.hip), FP64 ----
 struct LinearPredictorArgs {
   const double* luh;  // [cells][B^3][V+P]
-  double* lduh;       // [cells][B^3][V] volumeIntegralLinear of the prediction (may be null)
+  double* lduh;       // [cells][B^3][V] volumeIntegralLinear of the prediction (grid predictor only)
   double* lQhbnd;     // [cells][6][B^2][V+P]
-  double* lFhbnd;     // [cells][6][B^2][V]
+  double* lFhbnd;     // [cells][6][B^2][V] (not the grid predictor's)
   const double* dx;   // dx[cell * dx_stride + d]
   long dx_stride;
   const double* dt;   // device scalar
@@ -301,6 +298,10 @@ hipError_t launch_point_source(const SolverDesc& sd, double* PSi, const double* 
                                hipStream_t s);
 hipError_t launch_linear_predictor(const SolverDesc& sd, bool export_temps, const LinearPredictorArgs& a,
                                    long ncells, hipStream_t s);
+// The predictor of a linear grid: lduh and lQhbnd of every cell (its lFhbnd has
+// no reader: the linear Riemann solver takes the states).
+hipError_t launch_linear_grid_predictor(const SolverDesc& sd, const LinearPredictorArgs& a, long ncells,
+                                        hipStream_t s);
 // riemannSolverLinear over a face list (fluctuations into both cells' blocks)
 hipError_t launch_linear_riemann(const SolverDesc& sd, const RiemannArgs& a, hipStream_t s);
 // volumeIntegralLinear of one or more cells: lduh = -w^3 sum_d lFhi_d

@@ -242,3 +242,31 @@ def test_linear_elastic_2d_predictor_golden_on_device(exa, oracle):
     dt = 0.813172798364530
     o = exa.space_time_predictor_linear(s, luh.ravel(), dx, dt, temps=True)
     _check_stp_linear_elastic_golden(g, o["lQhi"], o["lFhi"], o["lQhbnd"], o["lFhbnd"])
+
+
+@pytest.mark.parametrize("order,n", [(2, (1, 3, 2)), (3, (5, 2, 9)), (4, (3, 4, 5)), (5, (2, 5, 1))])
+@pytest.mark.parametrize("boundary", ["periodic", "transmissive"])
+def test_linear_grid_uneven_vs_oracle(exa, oracle, order, n, boundary):
+    """The linear grid step on uneven grids (a side of one cell is its own
+    neighbour; a number of cells that is no multiple of eight) in a varying
+    material, from random states: one step against the oracle's grid driver."""
+    print(f"case: linear grid {n} N={order} {boundary}", flush=True)
+    rng = np.random.default_rng(order)
+    B3 = (order + 1) ** 3
+    cells = n[0] * n[1] * n[2]
+    luh = rng.uniform(-1, 1, (cells, B3, 12))
+    luh[..., 9:] = rng.uniform(1.0, 2.0, (cells, B3, 3))
+    s = oracle.elastic_solver(order)
+    s.linear = 1
+    o = oracle.Grid(s, n, transmissive=boundary == "transmissive")
+    o.set_solution(luh.ravel())
+    o.step(1)
+    g = exa.Grid(exa.elastic_solver(order, linear=True), n,
+                 boundary=exa.BC_TRANSMISSIVE if boundary == "transmissive" else exa.BC_PERIODIC)
+    g.upload(luh.ravel())
+    g.step(1)
+    got, want = g.solution().reshape(-1, 12), o.solution().reshape(-1, 12)
+    assert np.array_equal(got[:, 9:], luh.reshape(-1, 12)[:, 9:])  # the parameters stay
+    scale = np.abs(want).max(axis=0)
+    assert (np.abs(got - want).max(axis=0) <= 1e-12 * scale).all()
+    g.close()
