@@ -387,6 +387,11 @@ size_t predictor_ws_bytes_per_cell(const SolverDesc& sd, int variant) {
   size_t bytes = 0;
   (void)dispatch_pde(sd, [&]<int B, class PDE>() -> hipError_t {
     constexpr int V = PDE::V, D = PDE::V + PDE::P;
+    if constexpr (std::is_same_v<PDE, Elastic>) {  // no fluxes
+      bytes = sd.precision == kFP32Bulk ? PredictorLayout<B, V, D, true, float, 144, false>::ws_bytes
+                                        : PredictorLayout<B, V, D, true, double, 144, false>::ws_bytes;
+      return hipSuccess;
+    }
     if (variant == kPredictorValu64 && predictor_has_lds64(sd)) {
       bytes = sd.precision == kFP32Bulk ? PredictorLayout<B, V, D, false, float, 64>::ws_bytes
                                         : PredictorLayout<B, V, D, false, double, 64>::ws_bytes;

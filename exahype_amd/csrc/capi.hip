@@ -505,6 +505,10 @@ hipError_t launch_initial_dt(exa_grid* g) {
   });
 }
 
+// The one-kernel corrector of the library's PDEs without fluxes reads no lFhbnd
+// (a user's may: its boundary values can hold a flux).
+bool skips_zero_fluxes(const exa_grid* g) { return !(g->sd.terms & exa::kFlux) && g->fused_corrector && !g->user; }
+
 // The prediction with the time step size at dt (device scalar); run_if (a
 // device flag, may be null) gates the whole launch.
 hipError_t launch_predict(exa_grid* g, const double* dt, const int* run_if = nullptr) {
@@ -535,6 +539,7 @@ hipError_t launch_predict(exa_grid* g, const double* dt, const int* run_if = nul
   a.ws_cells = g->ws_cells;
   a.variant = g->predictor_variant;
   a.run_if = run_if;
+  a.skip_zero_fluxes = skips_zero_fluxes(g);
   hipError_t e = staged(g, EXA_STAGE_PREDICTOR, [&] {
     return g->user ? (hipError_t)g->user->predictor(&a, g->ncells, g->sd.precision, g->stream)
                    : exa::launch_predictor(g->sd, false, a, g->ncells, g->stream);
@@ -931,6 +936,10 @@ extern "C" int exa_grid_set_fused_corrector(exa_grid* g, int on) {
   if (on && g->sd.linear) return EXA_E_UNSUPPORTED;
   // boundary values and the per-step adjustment run in the one-kernel corrector
   if (!on && (g->boundary == exa::kBoundaryUser || g->adjust || g->user)) return EXA_E_UNSUPPORTED;
+  if (!on && g->lFhbnd && skips_zero_fluxes(g)) {  // the passes read the zeros the last prediction left out
+    const Sizes z(g->sd);
+    EXA_TRY(hipMemsetAsync(g->lFhbnd, 0, g->bulk * g->ncells * 6 * z.B2 * z.V, g->stream));
+  }
   g->fused_corrector = on != 0;
   return EXA_OK;
 }

@@ -21,13 +21,16 @@ static hipError_t launch_corrector_t(const SolverDesc& sd, const CorrectorArgs& 
   if (ELASTIC && !ncp) return hipErrorNotSupported;
   if (sd.precision == kFP32Bulk) {
     if (ncp) {
-      if constexpr (ELASTIC) hipLaunchKernelGGL((corrector_kernel<B, PDE, true, float>), grid, block, 0, s, a);
-      else return hipErrorNotSupported;
+      // no fluxes: lFhbnd is zero and not read (nor written, skip_zero_fluxes)
+      if constexpr (ELASTIC)
+        hipLaunchKernelGGL((corrector_kernel<B, PDE, true, float, false, false>), grid, block, 0, s, a);
+      else
+        return hipErrorNotSupported;
     } else {
       hipLaunchKernelGGL((corrector_kernel<B, PDE, false, float>), grid, block, 0, s, a);
     }
   } else if (ncp) {
-    hipLaunchKernelGGL((corrector_kernel<B, PDE, true, double>), grid, block, 0, s, a);
+    hipLaunchKernelGGL((corrector_kernel<B, PDE, true, double, false, !ELASTIC>), grid, block, 0, s, a);
   } else {
     hipLaunchKernelGGL((corrector_kernel<B, PDE, false, double>), grid, block, 0, s, a);
   }

@@ -122,7 +122,7 @@ void free_wave(Wave& w) {
   w.groups.clear();
 }
 
-exa::PredictorArgs pred_args(const Wave& w, const Group& g) {
+exa::PredictorArgs pred_args(const Wave& w, const Group& g, bool fused_corrector) {
   exa::PredictorArgs a{};
   a.luh = g.luh;
   a.lduh = g.lduh;
@@ -135,6 +135,8 @@ exa::PredictorArgs pred_args(const Wave& w, const Group& g) {
   a.ws_cells = g.ws_cells;
   a.cell_patch = g.cell_patch;
   a.variant = g.variant;
+  // the one-kernel corrector reads no lFhbnd of a PDE without fluxes
+  a.skip_zero_fluxes = fused_corrector && !(g.sd.terms & exa::kFlux);
   return a;
 }
 
@@ -217,7 +219,7 @@ hipError_t wave_step(const Wave& w, bool fused_corrector, hipStream_t s, StepTim
   for (size_t gi = 0; gi < w.groups.size(); ++gi) {
     const auto& g = w.groups[gi];
     if (e != hipSuccess) break;
-    e = tm.run(s, 0, (int)gi, [&] { return exa::launch_predictor(g.sd, false, pred_args(w, g), g.ncells, s); });
+    e = tm.run(s, 0, (int)gi, [&] { return exa::launch_predictor(g.sd, false, pred_args(w, g, fused_corrector), g.ncells, s); });
     if (e == hipSuccess && timer) e = exa::launch_count_iterations(g.iters, g.ncells, g.counters, s);
   }
   return e;
@@ -349,7 +351,7 @@ int build_wave(exa_patchset* b, const std::vector<int>& ids, Wave& w) {
   // first time step sizes and predictions
   for (const auto& g : w.groups) EXA_TRY(exa::launch_update(g.sd, 0, upd_args(w, g), g.ncells, b->stream));
   EXA_TRY(exa::launch_patch_dt_finalize(w.dt, w.t, w.slots, np, kSlotsPerPatch, false, b->stream));
-  for (const auto& g : w.groups) EXA_TRY(exa::launch_predictor(g.sd, false, pred_args(w, g), g.ncells, b->stream));
+  for (const auto& g : w.groups) EXA_TRY(exa::launch_predictor(g.sd, false, pred_args(w, g, b->fused_corrector), g.ncells, b->stream));
   EXA_TRY(hipStreamSynchronize(b->stream));
   return EXA_OK;
 }
@@ -369,9 +371,9 @@ int autotune(exa_patchset* b, Wave& w) {
     for (int v = 0; v < exa::kPredictorVariants; ++v) {
       if (!(variants & (1u << v))) continue;
       g.variant = v;
-      EXA_TRY(exa::launch_predictor(g.sd, false, pred_args(w, g), g.ncells, b->stream));  // warm-up
+      EXA_TRY(exa::launch_predictor(g.sd, false, pred_args(w, g, b->fused_corrector), g.ncells, b->stream));  // warm-up
       EXA_TRY(hipEventRecord(e0, b->stream));
-      for (int r = 0; r < 3; ++r) EXA_TRY(exa::launch_predictor(g.sd, false, pred_args(w, g), g.ncells, b->stream));
+      for (int r = 0; r < 3; ++r) EXA_TRY(exa::launch_predictor(g.sd, false, pred_args(w, g, b->fused_corrector), g.ncells, b->stream));
       EXA_TRY(hipEventRecord(e1, b->stream));
       EXA_TRY(hipEventSynchronize(e1));
       float ms = 0.f;
@@ -384,7 +386,7 @@ int autotune(exa_patchset* b, Wave& w) {
     g.variant = choice;
     b->variant_choice[g.pde][g.order] = choice;
     // leave the state as the chosen variant computes it
-    EXA_TRY(exa::launch_predictor(g.sd, false, pred_args(w, g), g.ncells, b->stream));
+    EXA_TRY(exa::launch_predictor(g.sd, false, pred_args(w, g, b->fused_corrector), g.ncells, b->stream));
   }
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);

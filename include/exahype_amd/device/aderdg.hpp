@@ -97,6 +97,9 @@ struct PredictorArgs {
   // optional gate for the whole launch: it does nothing unless *run_if != 0
   // (the fused time stepping's re-run after a violated stability condition)
   const int* run_if;
+  // PDEs without fluxes: leave lFhbnd, identically zero, unwritten (the caller's
+  // corrector does not read it)
+  int skip_zero_fluxes;
 };
 
 struct RiemannArgs {

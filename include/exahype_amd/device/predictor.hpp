@@ -28,7 +28,9 @@ constexpr float kPicardRelTol32 = 1e-6f;
 
 // S = algebraicSource(Q) - NCP(Q, gradQ) at node (z,y,x) of a time slice whose
 // variables are staged in sQ[var][node] (spaceTimePredictorNonlinear.cpph:238-266).
-template <int B, class PDE, bool USE_SOURCE, bool USE_NCP, typename T>
+// ONE_LINE: one variable's line entries at a time in registers (otherwise the
+// reads of all variables go out together, which takes most of the registers).
+template <int B, class PDE, bool USE_SOURCE, bool USE_NCP, bool ONE_LINE, typename T>
 __device__ inline void source_ncp(const T* Q, const T* sQ, const T* sDu, const T invDx[3], int z, int y,
                                   int x, T* S) {
   constexpr int V = PDE::V;
@@ -40,20 +42,21 @@ __device__ inline void source_ncp(const T* Q, const T* sQ, const T* sDu, const T
     for (int m = 0; m < V; ++m) S[m] = T(0);
   }
   if (USE_NCP) {
-    // gradQ(dir, var) = sum_n invDx * lQi(..n..) * dudx[l][n] (:170-173, 199-202, 228-231)
+    // gradQ(dir, var) = invDx * sum_n lQi(..n..) * dudx[l][n] (:170-173, 199-202, 228-231)
     T gradQ[3][V];
 #pragma unroll
     for (int m = 0; m < V; ++m) {
       T gx = T(0), gy = T(0), gz = T(0);
 #pragma unroll
       for (int n = 0; n < B; ++n) {
-        gx += T(1) * invDx[0] * sQ[m * B3 + (z * B + y) * B + n] * sDu[x * B + n];
-        gy += T(1) * invDx[1] * sQ[m * B3 + (z * B + n) * B + x] * sDu[y * B + n];
-        gz += T(1) * invDx[2] * sQ[m * B3 + (n * B + y) * B + x] * sDu[z * B + n];
+        gx += sQ[m * B3 + (z * B + y) * B + n] * sDu[x * B + n];
+        gy += sQ[m * B3 + (z * B + n) * B + x] * sDu[y * B + n];
+        gz += sQ[m * B3 + (n * B + y) * B + x] * sDu[z * B + n];
       }
-      gradQ[0][m] = gx;
-      gradQ[1][m] = gy;
-      gradQ[2][m] = gz;
+      gradQ[0][m] = invDx[0] * gx;
+      gradQ[1][m] = invDx[1] * gy;
+      gradQ[2][m] = invDx[2] * gz;
+      if (ONE_LINE) __builtin_amdgcn_sched_barrier(0);
     }
     T ncp[V];
     PDE::ncp(Q, gradQ, ncp);
@@ -68,17 +71,26 @@ __device__ inline void source_ncp(const T* Q, const T* sQ, const T* sDu, const T
 // registers or, when registers run out (WSQ), in a per-cell device workspace
 // that each thread reads and writes only at its own nodes.  Large sizes run
 // the loop over time slices rolled (ROLLED).
-template <int B, int V, int D, bool USE_NCP, typename T, int LDSK = 144>
+// A PDE without fluxes whose slices all fit LDS takes the gradients from the
+// iterate itself (IN_PLACE): no staged copy, no flux rows, and no barrier
+// between slices, which only read the iterate.  In double at N=4 a cell takes
+// 45 KB of LDS instead of 81, so three workgroups of two wavefronts per CU
+// instead of one; LDS reads of the gradients' lines bound it.  Elastic N=4 in
+// double, 41^3 cells, 8 steps: predictor 4.08 -> 2.26 ms per step together
+// with the closed first iteration, the whole run 51.1 -> 46.7 ms by this form
+// and the boundary fluxes left out.
+template <int B, int V, int D, bool USE_NCP, typename T, int LDSK = 144, bool USE_FLUX = true>
 struct PredictorLayout {
   static constexpr int B2 = B * B, B3 = B2 * B;
   static constexpr int NT = node_threads(B);
   static constexpr bool IS_FP64 = sizeof(T) == sizeof(double);
-  // LDS: one slice of fluxes [dir][var][node] (reused for lQhi / lFhi staging)
-  static constexpr int SF = (3 * V > D ? 3 * V : D) * B3;
   static constexpr long kLdsBudget = (long)LDSK * 1024;
+  static constexpr bool IN_PLACE = USE_NCP && !USE_FLUX && (long)(B * V * B3 + B2 + 64) * (long)sizeof(T) <= kLdsBudget;
+  // LDS: one slice of fluxes [dir][var][node] (reused for lQhi / lFhi staging)
+  static constexpr int SF = IN_PLACE ? 0 : (3 * V > D ? 3 * V : D) * B3;
   static constexpr long kSliceBytes = (long)V * B3 * sizeof(T);
   static constexpr long kOther =
-      (long)(SF + (USE_NCP ? V * B3 + B2 : 0) + 3 + 2 * (NT / kWave)) * sizeof(T);
+      (long)(SF + (USE_NCP ? (IN_PLACE ? 0 : V * B3) + B2 : 0) + 3 + 2 * (NT / kWave)) * sizeof(T);
   static constexpr long kFree = kLdsBudget - kOther;
   static constexpr int NQL = kFree <= 0 ? 0 : (kFree / kSliceBytes >= B ? B : (int)(kFree / kSliceBytes));
   static constexpr int NQR = B - NQL;
@@ -119,15 +131,19 @@ struct PredictorLayout {
 // Waves per SIMD the register allocation must leave room for: the float
 // flux-only form at N=5 and N=7 accumulates its time-averaged fluxes during
 // the last iteration (3V more live registers) within the four (N=5) or three
-// (N=7, 64 KB layout) waves that its LDS allows anyway; elsewhere no
+// (N=7, 64 KB layout) waves that its LDS allows anyway; the elastic PDE, whose
+// next iterate alone takes 9 B registers or twice that, keeps the wavefronts
+// that its LDS allows (without the cap the compiler moves the line reads of
+// all variables to the front and one wavefront per SIMD is left); elsewhere no
 // constraint.
-template <int B, int TERMS, typename T>
+template <int B, class PDE, int TERMS, bool EXPORT, typename T>
 __host__ __device__ constexpr int predictor_min_waves() {
+  if (std::is_same_v<PDE, Elastic>) return sizeof(T) == sizeof(double) ? (B <= 5 && !EXPORT ? 2 : 1) : (B <= 5 ? 3 : 2);
   return (sizeof(T) == sizeof(float) && TERMS == kFlux) ? (B == 6 ? 4 : (B == 8 ? 3 : 1)) : 1;
 }
 
 template <int B, class PDE, int TERMS, bool EXPORT, typename T, int LDSK = 144>
-__global__ __launch_bounds__(node_threads(B), (predictor_min_waves<B, TERMS, T>())) void predictor_kernel(
+__global__ __launch_bounds__(node_threads(B), (predictor_min_waves<B, PDE, TERMS, EXPORT, T>())) void predictor_kernel(
     PredictorArgs a) {
   constexpr int V = PDE::V, P = PDE::P, D = V + P;
   constexpr int N = B - 1;
@@ -139,13 +155,16 @@ __global__ __launch_bounds__(node_threads(B), (predictor_min_waves<B, TERMS, T>(
   constexpr bool USE_SRC_NCP = USE_SOURCE || USE_NCP;
   constexpr bool IS_FP64 = sizeof(T) == sizeof(double);
   constexpr int MAX_ITER = 2 * B;  // spaceTimePredictorNonlinear.cpph:85
-  using L = PredictorLayout<B, V, D, USE_NCP, T, LDSK>;
-  constexpr int SF = L::SF, NQL = L::NQL, NQR = L::NQR, UNROLL_T = L::UNROLL_T;
+  using L = PredictorLayout<B, V, D, USE_NCP, T, LDSK, USE_FLUX>;
+  constexpr int NQL = L::NQL, NQR = L::NQR, UNROLL_T = L::UNROLL_T;
+  constexpr bool IN_PLACE = L::IN_PLACE;
+  static_assert(!IN_PLACE || (NQL == B && B * V >= D), "the iterate's rows hold the epilogue's D");
   constexpr bool SPLIT = L::SPLIT;
   constexpr bool WSQ = L::WSQ;
-  __shared__ T sF[SF];
+  __shared__ T sStage[IN_PLACE ? 1 : L::SF];
   __shared__ T sQi[NQL > 0 ? NQL * V * B3 : 1];  // lQi^k slices t < NQL, [t][var][node]
-  __shared__ T sQ[USE_NCP ? V * B3 : 1];
+  __shared__ T sQ[USE_NCP && !IN_PLACE ? V * B3 : 1];
+  T* const sF = IN_PLACE ? sQi : sStage;  // IN_PLACE: the epilogue's rows, when the iterate is done
   __shared__ T sDu[USE_NCP ? B2 : 1];  // dudx[l][n]
   __shared__ T sRed[2 * (NT / kWave)];
 
@@ -177,6 +196,10 @@ __global__ __launch_bounds__(node_threads(B), (predictor_min_waves<B, TERMS, T>(
   const double* dxp = a.cell_patch ? a.dx + (size_t)patch * 3 : a.dx + cell * a.dx_stride;
   const T invDx[3] = {T(1.0) / T(dxp[0]), T(1.0) / T(dxp[1]), T(1.0) / T(dxp[2])};
   const T dt = T(a.dt[patch]);
+  // the node's weights, for the volume integral; IN_PLACE has no registers to
+  // keep them through the iterations and takes them again afterwards
+  T wx = tc<T>(exa_gl_weights[N][x]), wy = tc<T>(exa_gl_weights[N][y]), wz = tc<T>(exa_gl_weights[N][z]);
+  T w3 = wz * wy * wx;
 
   T q0[D];
   {
@@ -184,8 +207,6 @@ __global__ __launch_bounds__(node_threads(B), (predictor_min_waves<B, TERMS, T>(
 #pragma unroll
     for (int m = 0; m < D; ++m) q0[m] = T(luh[m]);
   }
-  const T wx = tc<T>(exa_gl_weights[N][x]), wy = tc<T>(exa_gl_weights[N][y]), wz = tc<T>(exa_gl_weights[N][z]);
-  const T w3 = wz * wy * wx;  // weight of rhs0 (:130-132) and of iK1 (:286-288)
 
   // Picard state: the current iterate lQi^k of this node (in LDS, each thread
   // touching only its own node's entries so no barriers are needed, or in
@@ -286,18 +307,24 @@ __global__ __launch_bounds__(node_threads(B), (predictor_min_waves<B, TERMS, T>(
 
 #pragma unroll 1
   for (int iter = 0; iter < MAX_ITER; ++iter) {
+    T q0i[V];
     // FLCoeff[t] luh is loop invariant; keeping B V copies of it live across
     // iterations costs more registers than recomputing it per slice.
-    T q0i[V];
+    // IN_PLACE, whose next iterate takes most of the registers: luh is read
+    // again (L1, L2) and its share sum_t iK1[l][t] FLCoeff[t] luh starts the
+    // sums instead.
+    if constexpr (IN_PLACE) {
+      const double* luh = a.luh + cell * (size_t)(B3 * D) + node * D;
+      asm volatile("" : "+v"(luh));
 #pragma unroll
-    for (int m = 0; m < V; ++m) {
-      q0i[m] = q0[m];
-      asm volatile("" : "+v"(q0i[m]));
+      for (int m = 0; m < V; ++m) q0i[m] = T(luh[m]);
+    } else {
+#pragma unroll
+      for (int m = 0; m < V; ++m) {
+        q0i[m] = q0[m];
+        asm volatile("" : "+v"(q0i[m]));
+      }
     }
-#pragma unroll
-    for (int l = 0; l < B; ++l)
-#pragma unroll
-      for (int m = 0; m < V; ++m) qn[l][m] = T(0);
     if constexpr (ACC_FH) {
 #pragma unroll
       for (int d = 0; d < 3; ++d)
@@ -347,11 +374,11 @@ __global__ __launch_bounds__(node_threads(B), (predictor_min_waves<B, TERMS, T>(
           }
         }
       }
-      if (USE_NCP) {
+      if (USE_NCP && !IN_PLACE) {
 #pragma unroll
         for (int m = 0; m < V; ++m) sQ[m * B3 + node] = Q[m];
       }
-      __syncthreads();
+      if (!IN_PLACE) __syncthreads();
 
       if (USE_FLUX) contract_lines.template operator()<false>();
 
@@ -363,7 +390,7 @@ __global__ __launch_bounds__(node_threads(B), (predictor_min_waves<B, TERMS, T>(
       const T wg[3] = {wt * gd[0], wt * gd[1], wt * gd[2]};
 #pragma unroll
       for (int m = 0; m < V; ++m) {
-        ir[m] = fl_t * q0i[m];
+        ir[m] = IN_PLACE ? T(0) : fl_t * q0i[m];
         if (USE_FLUX) {
           ir[m] -= wg[0] * sF[(0 * V + m) * B3 + node];
           ir[m] -= wg[1] * sF[(1 * V + m) * B3 + node];
@@ -372,7 +399,7 @@ __global__ __launch_bounds__(node_threads(B), (predictor_min_waves<B, TERMS, T>(
       }
       if (USE_SRC_NCP) {
         T S[V];
-        source_ncp<B, PDE, USE_SOURCE, USE_NCP>(Q, sQ, sDu, invDx, z, y, x, S);
+        source_ncp<B, PDE, USE_SOURCE, USE_NCP, IN_PLACE>(Q, IN_PLACE ? sQi + t * (V * B3) : sQ, sDu, invDx, z, y, x, S);
         const T us = wt * dt;
 #pragma unroll
         for (int m = 0; m < V; ++m) ir[m] += us * S[m];
@@ -391,7 +418,8 @@ __global__ __launch_bounds__(node_threads(B), (predictor_min_waves<B, TERMS, T>(
       for (int m = 0; m < V; ++m)
 #pragma unroll
         for (int l = 0; l < B; ++l) qn[l][m] += ir[m] * tc<T>(exa_ik1[N][l][t]);
-      if (USE_FLUX || USE_NCP) __syncthreads();  // the next slice rewrites sF / sQ
+      if (USE_FLUX || (USE_NCP && !IN_PLACE)) __syncthreads();  // the next slice rewrites sF / sQ
+      if (IN_PLACE) __builtin_amdgcn_sched_barrier(0);  // one slice's reads at a time in registers
     };
     if (FIRST_CLOSED && iter == 0) {
       // Every slice of the initial iterate equals luh, so one evaluation
@@ -419,11 +447,11 @@ __global__ __launch_bounds__(node_threads(B), (predictor_min_waves<B, TERMS, T>(
             if constexpr (ACC_FH) fh[d][m] = F[d][m] * sumw;
           }
       }
-      if constexpr (USE_NCP) {
+      if constexpr (USE_NCP && !IN_PLACE) {
 #pragma unroll
         for (int m = 0; m < V; ++m) sQ[m * B3 + node] = Q[m];
       }
-      __syncthreads();
+      if constexpr (!IN_PLACE) __syncthreads();
       if constexpr (USE_FLUX) contract_lines.template operator()<false>();
 #pragma unroll
       for (int m = 0; m < V; ++m)
@@ -432,7 +460,7 @@ __global__ __launch_bounds__(node_threads(B), (predictor_min_waves<B, TERMS, T>(
                         : T(0);
       if constexpr (USE_SRC_NCP) {
         T S[V];
-        source_ncp<B, PDE, USE_SOURCE, USE_NCP>(Q, sQ, sDu, invDx, z, y, x, S);
+        source_ncp<B, PDE, USE_SOURCE, USE_NCP, IN_PLACE>(Q, IN_PLACE ? sQi : sQ, sDu, invDx, z, y, x, S);
 #pragma unroll
         for (int m = 0; m < V; ++m) {
           R[m] -= dt * S[m];
@@ -444,17 +472,22 @@ __global__ __launch_bounds__(node_threads(B), (predictor_min_waves<B, TERMS, T>(
 #pragma unroll
         for (int m = 0; m < V; ++m)
           qn[l][m] = tc<T>(exa_folded.a[N][l]) * q0i[m] - tc<T>(exa_folded.b[N][l]) * R[m];
-      __syncthreads();  // the next iteration rewrites sF / sQ
-    } else if constexpr (SPLIT) {
-#pragma unroll 1
-      for (int t = 0; t < NQL; ++t) picard_slice(t);
-#pragma unroll 1
-      for (int t = NQL; t < B; ++t) picard_slice(t);
+      if constexpr (!IN_PLACE) __syncthreads();  // the next iteration rewrites sF / sQ
     } else {
+#pragma unroll
+      for (int l = 0; l < B; ++l)
+#pragma unroll
+        for (int m = 0; m < V; ++m) qn[l][m] = IN_PLACE ? tc<T>(exa_folded.a[N][l]) * q0i[m] : T(0);
+      if constexpr (SPLIT) {
+#pragma unroll 1
+        for (int t = 0; t < NQL; ++t) picard_slice(t);
+#pragma unroll 1
+        for (int t = NQL; t < B; ++t) picard_slice(t);
+      } else {
 #pragma unroll UNROLL_T
-      for (int t = 0; t < B; ++t) picard_slice(t);
+        for (int t = 0; t < B; ++t) picard_slice(t);
+      }
     }
-
     // squared residual (:303) and exit test (:314-318)
     T sq = T(0), qq = T(0);
 #pragma unroll
@@ -464,6 +497,7 @@ __global__ __launch_bounds__(node_threads(B), (predictor_min_waves<B, TERMS, T>(
         const T dq = qn[l][m] - qi(l, m);
         sq += dq * dq;
         if (!IS_FP64) qq += qn[l][m] * qn[l][m];
+        if (IN_PLACE && m + 1 == V) __builtin_amdgcn_sched_barrier(0);  // one slice's reads at a time in registers
       }
     if (!active) {
       sq = T(0);
@@ -482,11 +516,24 @@ __global__ __launch_bounds__(node_threads(B), (predictor_min_waves<B, TERMS, T>(
       iters = iter + 1;
       break;  // qi still holds lQi^k, the iterate the last fluxes were taken from
     }
+    if constexpr (IN_PLACE) __syncthreads();  // every gradient of the iterate is taken
 #pragma unroll
     for (int l = 0; l < B; ++l)
 #pragma unroll
       for (int m = 0; m < V; ++m)
         qi_set(l, m, qn[l][m]);
+    if constexpr (IN_PLACE) __syncthreads();
+  }
+  int own = node;
+  if constexpr (IN_PLACE) {
+    __syncthreads();  // the residual has read the iterate
+    own = threadIdx.x;
+    asm volatile("" : "+v"(own));
+    own = own < B3 ? own : 0;
+    wx = tc<T>(exa_gl_weights[N][own % B]);
+    wy = tc<T>(exa_gl_weights[N][(own / B) % B]);
+    wz = tc<T>(exa_gl_weights[N][own / B2]);
+    w3 = wz * wy * wx;
   }
 
   // ---- epilogue: time average, extrapolation, volume integral ----
@@ -584,7 +631,7 @@ __global__ __launch_bounds__(node_threads(B), (predictor_min_waves<B, TERMS, T>(
       }
       if (USE_NCP) __syncthreads();
       T S[V];
-      source_ncp<B, PDE, USE_SOURCE, USE_NCP>(Q, sQ, sDu, invDx, z, y, x, S);
+      source_ncp<B, PDE, USE_SOURCE, USE_NCP, IN_PLACE>(Q, sQ, sDu, invDx, z, y, x, S);
 #pragma unroll
       for (int m = 0; m < V; ++m) sh[m] += S[m] * wt;
       if (USE_NCP) __syncthreads();
@@ -613,15 +660,17 @@ __global__ __launch_bounds__(node_threads(B), (predictor_min_waves<B, TERMS, T>(
       lFhi[3 * B3 * V + ((z * B + y) * B + x) * V + m] = sh[m];
     }
   }
+  if constexpr (USE_FLUX) {
 #pragma unroll
-  for (int d = 0; d < 3; ++d)
+    for (int d = 0; d < 3; ++d)
 #pragma unroll
-    for (int m = 0; m < V; ++m) sF[(d * V + m) * B3 + node] = fh[d][m];
-  __syncthreads();
+      for (int m = 0; m < V; ++m) sF[(d * V + m) * B3 + node] = fh[d][m];
+    __syncthreads();
+  }
   // lFhbnd from lFhi_{x,y,z} (:434-527)
   if (USE_FLUX) {
     extrapolate.template operator()<V, true>(out_lFhbnd, cFb);
-  } else {
+  } else if (!a.skip_zero_fluxes) {
 #pragma unroll 1
     for (int round = 0; round < (6 * B2 * V + NT - 1) / NT; ++round)
       out_lFhbnd[cFb + min(tid + round * NT, 6 * B2 * V - 1)] = T(0);
@@ -646,7 +695,7 @@ __global__ __launch_bounds__(node_threads(B), (predictor_min_waves<B, TERMS, T>(
 #pragma unroll
       for (int m = 0; m < V; ++m) acc[m] += w3 * sh[m];
     }
-    T* lduh = out_lduh + cell * (size_t)(B3 * V) + node * V;
+    T* lduh = out_lduh + cell * (size_t)(B3 * V) + own * V;
 #pragma unroll
     for (int m = 0; m < V; ++m) lduh[m] = acc[m];
   }
