@@ -10,6 +10,7 @@
 //   euler_ic_kernel, elastic_ic_kernel               the workloads' initial conditions
 #include "corrector.hpp"
 #include "predictor.hpp"
+#include "predictor_wave.hpp"
 #include "aderdg.hpp"
 #include "exa_device.hpp"
 
@@ -312,6 +313,14 @@ static hipError_t dispatch_pde(const SolverDesc& sd, F&& f) {
   return hipErrorNotSupported;
 }
 
+// The size that Auto runs with one wavefront per time slice (predictor_wave.hpp
+// says why this one, with the measurements of the others).
+constexpr int kSliceWaveB = 7;
+static bool predictor_by_slices(const SolverDesc& sd, int variant) {
+  return variant == kPredictorAuto && sd.pde == kPdeEuler && sd.npar == 0 && sd.terms == kFlux &&
+         sd.order + 1 == kSliceWaveB;
+}
+
 hipError_t launch_predictor(const SolverDesc& sd, bool export_temps, const PredictorArgs& a, long ncells,
                             hipStream_t s) {
   if (ncells <= 0) return hipSuccess;
@@ -320,7 +329,7 @@ hipError_t launch_predictor(const SolverDesc& sd, bool export_temps, const Predi
     if (export_temps) return hipErrorNotSupported;
     return launch_predictor_mfma(sd, a, ncells, s);
   }
-  const size_t ws = predictor_ws_bytes_per_cell(sd, a.variant);
+  const size_t ws = predictor_ws_bytes_per_cell(sd, export_temps ? (int)kPredictorValu144 : a.variant);
   if (ws > 0 && (a.ws == nullptr || a.ws_cells <= 0)) return hipErrorInvalidValue;
   const long chunk = ws > 0 ? a.ws_cells : ncells;
   return dispatch_pde(sd, [&]<int B, class PDE>() -> hipError_t {
@@ -337,6 +346,13 @@ hipError_t launch_predictor(const SolverDesc& sd, bool export_temps, const Predi
           hipLaunchKernelGGL((predictor_kernel<B, PDE, kNCP, true, double>), grid, block, 0, s, ac);
         else
           hipLaunchKernelGGL((predictor_kernel<B, PDE, kNCP, false, double>), grid, block, 0, s, ac);
+      } else if (!export_temps && predictor_by_slices(sd, a.variant)) {
+        if constexpr (B == kSliceWaveB && PDE::P == 0) {
+          if (sd.precision == kFP32Bulk)
+            hipLaunchKernelGGL((predictor_wave_kernel<B, PDE, float>), grid, dim3(B * kWave), 0, s, ac);
+          else
+            hipLaunchKernelGGL((predictor_wave_kernel<B, PDE, double>), grid, dim3(B * kWave), 0, s, ac);
+        }
       } else if (sd.precision == kFP32Bulk) {
         if (sd.terms != kFlux) return hipErrorNotSupported;
         if (a.variant == kPredictorValu64 && PDE::P == 0)
@@ -385,6 +401,7 @@ bool predictor_variant_available(const SolverDesc& sd, int variant) {
 
 size_t predictor_ws_bytes_per_cell(const SolverDesc& sd, int variant) {
   size_t bytes = 0;
+  if (predictor_by_slices(sd, variant)) return 0;
   (void)dispatch_pde(sd, [&]<int B, class PDE>() -> hipError_t {
     constexpr int V = PDE::V, D = PDE::V + PDE::P;
     if constexpr (std::is_same_v<PDE, Elastic>) {  // no fluxes

@@ -89,7 +89,7 @@ static int predictor_impl(const exa_solver* s, long ncells, double* lQhbnd, doub
   a.lQhi = d_qhi.d();
   a.lFhi = d_fhi.d();
   DevBuf d_ws;
-  if (const size_t wsb = exa::predictor_ws_bytes_per_cell(sd)) {
+  if (const size_t wsb = exa::predictor_ws_bytes_per_cell(sd, exp ? exa::kPredictorValu144 : exa::kPredictorAuto)) {
     a.ws_cells = std::min(ncells, exa::kPredictorWsCells);
     EXA_TRY(d_ws.alloc(wsb * a.ws_cells));
     a.ws = d_ws.p;

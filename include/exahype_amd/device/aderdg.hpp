@@ -228,9 +228,10 @@ bool supported_sizes(const SolverDesc& sd);
 hipError_t launch_predictor(const SolverDesc& sd, bool export_temps, const PredictorArgs& a,
                             long ncells, hipStream_t s);
 // Predictor variants.  kPredictorAuto: the measured default, the vector-ALU
-// kernel (predictor_kernel) with its 144 KB LDS budget; kPredictorValu64 /
-// kPredictorValu144: that kernel with a 64 KB / 144 KB LDS budget for the
-// Picard iterate (see PredictorLayout); kPredictorMfma: the FP32-bulk kernel
+// kernel (predictor_kernel) with its 144 KB LDS budget or, at the size where it
+// is faster, the one with a wavefront per time slice (predictor_wave.hpp);
+// kPredictorValu64 / kPredictorValu144: predictor_kernel with a 64 KB / 144 KB
+// LDS budget for the Picard iterate (see PredictorLayout); kPredictorMfma: the FP32-bulk kernel
 // with its contractions on the matrix cores (predictor_mfma.hip), where
 // compiled (predictor_mfma_supported).
 enum : int { kPredictorAuto = 0, kPredictorValu64 = 1, kPredictorValu144 = 2, kPredictorMfma = 3 };
@@ -238,7 +239,8 @@ constexpr int kPredictorVariants = 4;
 // Bytes of PredictorArgs::ws one cell needs (0: no workspace), for a variant.
 size_t predictor_ws_bytes_per_cell(const SolverDesc& sd, int variant = kPredictorAuto);
 // Bit v set: variant v runs a kernel of its own for this solver (bit 0 always;
-// kPredictorValu144 is the Auto kernel, so its bit is never set).
+// kPredictorValu144 is the Auto kernel or the slower of the two, so its bit is
+// never set).
 unsigned predictor_variants(const SolverDesc& sd);
 // Whether a variant can be requested for this solver (it may share Auto's kernel).
 bool predictor_variant_available(const SolverDesc& sd, int variant);

@@ -87,6 +87,34 @@ def test_matrix_core_predictor_vs_vector_alu(exa, order, n):
     assert abs(its[exa.PREDICTOR_MFMA] - its[exa.PREDICTOR_AUTO]) <= 0.1
 
 
+@pytest.mark.parametrize("fused", [False, True])
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("n", [1, (3, 2, 5)])
+def test_slice_wavefront_predictor_vs_node_threads(exa, precision, n, fused):
+    """Order 6: the predictor with a wavefront per time slice (AUTO) against the
+    one with a thread per node (VALU_LDS144).  Same sums in another order: the
+    bars of the corrector's two forms, FP64 1e-13 and FP32-bulk 1e-6 relative
+    L2 after 5 steps; FP64 takes the same Picard iterations."""
+    print(f"case: order 6 predictor forms, {n}, precision {precision}, fused {fused}", flush=True)
+    out = []
+    for variant in (exa.PREDICTOR_AUTO, exa.PREDICTOR_VALU_LDS144):
+        g = exa.Grid(exa.euler_solver(6, precision=precision), n)
+        g.set_predictor_variant(variant)
+        g.init_euler(nmodes=8, mode_amp=0.05, seed=4)
+        if fused:
+            g.set_fused_time_stepping(True)
+        g.set_profiling(True)
+        g.step(5)
+        out.append((g.solution(), g.picard_totals()))
+        g.close()
+    (a, ia), (b, ib) = out
+    l2 = np.linalg.norm(a - b) / np.linalg.norm(b)
+    print(f"  L2 {l2:.2e} picard {ia} {ib}", flush=True)
+    assert l2 < (1e-13 if precision == 0 else 1e-6)
+    if precision == 0:
+        assert ia == ib
+
+
 def test_predictor_variant_setter_rejects_unsupported(exa):
     """Variants the solver does not compile are refused (the FP64 form has no
     matrix-core kernel); out-of-range values are invalid."""
