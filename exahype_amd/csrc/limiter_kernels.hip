@@ -30,6 +30,7 @@
 #include "exa_device.hpp"
 #include "fv_device.hpp"
 #include "limiter.hpp"
+#include "line_ops.hpp"
 
 namespace exa {
 
@@ -38,7 +39,6 @@ __constant__ LimTables c_lim;
 static unsigned blocks256(long n) { return (unsigned)((n + 255) / 256); }
 
 constexpr int kLimNT = 256;     // per-cell kernels
-constexpr int kMusclNT = 448;   // MUSCL-Hancock patch kernel (LDS allows one per CU; seven wavefronts)
 
 template <int N>
 struct LimShape {
@@ -53,8 +53,8 @@ struct LimShape {
 // out[v][Z][Y][X] = sum in[v][z][y][x] T[z][Z] T[y][Y] T[x][X]; in/out/t1/t2
 // in LDS, T (P x M, row = input index) in LDS.  Ends with a barrier.
 template <int P, int M, int V, int NT>
-__device__ inline void tensor3(const double* in, const double* T, double* t1, double* t2, double* out) {
-  const int tid = threadIdx.x;
+__device__ inline void tensor3(const double* in, const double* T, double* t1, double* t2, double* out,
+                               const int tid = threadIdx.x) {
   for (int i = tid; i < V * P * P * M; i += NT) {  // t1[v][z][y][X]
     const int X = i % M, r = i / M;
     const double* row = in + r * P;
@@ -311,173 +311,235 @@ __global__ __launch_bounds__(kLimNT) void lim_ghost_kernel(LimArgs a, int only_i
 // GODUNOV: the first-order update (GOD:35-143) -- the face states are the
 // cell values themselves, the face fluxes and their accumulation order are
 // those of MUSCL-Hancock (the two reference kernels share both).
+//
+// One thread per interior cell, and one per face line on top: a direction at a
+// time, the left states of its faces are in LDS, a thread forms the flux of the
+// face below its cell (the last L^2 threads the topmost faces) over the left
+// state, and the cells on both sides take it from there.  The ghost cells'
+// states are formed once, by the last wavefronts, beside the interior's
+// evolution.  So a patch takes 81 KB of LDS (N=3) and seven wavefronts, two
+// workgroups per CU within 128 registers; the states of all directions and both
+// sides took 147 KB, one workgroup per CU.  Bound by FP64 issue and the
+// barriers of a direction (three each).  Blast wave, one launch (MUSCL-Hancock):
+//   N=3, 63x60x55 cells: 0.99 -> 0.55 ms;  N=2, 15^3 cells: 77 -> 43 us.
+// (A thread per evolved cell, ten wavefronts a patch: 0.86 ms and 54 us -- dealt
+// three to two SIMDs, a second workgroup of 96 registers does not fit.)
 // ---------------------------------------------------------------------------
-template <int N, bool GODUNOV>
-__global__ __launch_bounds__(kMusclNT) void lim_fv_update_kernel(LimArgs a, int only_if_irregular) {
+template <int N>
+struct MusclShape {
+  using Sh = LimShape<N>;
+  static constexpr int L2 = Sh::L * Sh::L;
+  static constexpr int NF = L2 * (Sh::L + 1);  // faces per direction
+  static constexpr int NT = (NF + kWave - 1) / kWave * kWave;
+  static_assert(6 * L2 <= NT, "one ghost cell per thread");
+  // workgroups per CU, by LDS (160 KB) and by four wavefronts per SIMD
+  static constexpr int kLds = (Sh::PATCH + Sh::V * (NF + 6 * L2) + Sh::L * Sh::B + 2 * Sh::V * (NT / kWave)) * 8;
+  static constexpr int kPerCu = 160 * 1024 / kLds < 16 / (NT / kWave) ? 160 * 1024 / kLds : 16 / (NT / kWave);
+};
+
+template <int N, bool GODUNOV, bool DT_MAX>
+__global__ __launch_bounds__(MusclShape<N>::NT, (DT_MAX ? 2 : 4)) void lim_fv_update_kernel(LimArgs a, int only_if_irregular) {
   using Sh = LimShape<N>;
   constexpr int L = Sh::L, G = Sh::G, S = Sh::S, V = Sh::V, PATCH = Sh::PATCH, L3 = Sh::L3, B = Sh::B;
-  constexpr int NF = L * L * (L + 1);  // faces per direction
-  constexpr int NC = L3 + 6 * L * L;   // cells to evolve
+  constexpr int NF = MusclShape<N>::NF, L2 = L * L, NT = MusclShape<N>::NT, NW = NT / kWave;
+  constexpr int T1 = V * L3, T2 = T1 + V * L * L * B, OUT = T2 + V * L * B * B;  // the projection's rows in sP
+  static_assert(OUT + V * Sh::B3 <= PATCH);
   __shared__ double sP[PATCH];
-  __shared__ double sF[3 * 2 * V * NF];  // [d][side][v][a][b][f]; flux into side 0
+  __shared__ double sX[V * NF];  // [v][z][y][x] of a direction's faces: left states, then fluxes
+  __shared__ double sG[V * 6 * L2];  // [v][sheet][r]: the ghost cells' states
   __shared__ double sLim2uh[L * B];
-  __shared__ double red[2 * V * (kMusclNT / kWave)];
+  __shared__ double red[2 * V * NW];
   if (only_if_irregular && !a.flags[kLimFlagIrregular]) return;
   load_tables<N>(nullptr, nullptr, sLim2uh);
   const int count = a.flags[kLimFlagFvCount];
   const double dt = a.st_state->dt;
-  const double h[3] = {a.dx[0] / L, a.dx[1] / L, a.dx[2] / L};
-  const double ih[3] = {1. / h[0], 1. / h[1], 1. / h[2]};
-  const double cdt[3] = {dt * ih[0], dt * ih[1], dt * ih[2]};
-  auto fidx = [](int d, int side, int v, int fa, int fb, int f) {
-    return ((((d * 2 + side) * V + v) * L + fa) * L + fb) * (L + 1) + f;
-  };
+  double h[3], hh[3], ih[3], cdt[3];  // in scalar registers
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    h[d] = wave_uniform(a.dx[d] / L);
+    hh[d] = wave_uniform(0.5 * h[d]);
+    ih[d] = wave_uniform(1. / h[d]);
+    cdt[d] = wave_uniform(dt * ih[d]);
+  }
+  const double hdt = wave_uniform(0.5 * dt);
+  const int step[3] = {1, S, S * S};
+  double dt_allowed = DBL_MAX;  // min over faces of cflFactor/3 h_d / s_max (MH:267-329); FV solver CFL / MH:29
   for (int it = blockIdx.x; it < count; it += gridDim.x) {
-    const int c = a.fv_list[it];
-    const int ob = a.cur[c];
+    const int c = wave_uniform(a.fv_list[it]);
+    const int ob = wave_uniform((int)a.cur[c]);
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));  // its index arithmetic stays where it is used: no registers held for it
     const double* old = patch_ptr(a, c, ob, PATCH);
     double* nw = patch_ptr(a, c, ob ^ 1, PATCH);
-    __syncthreads();  // the previous patch's LDS use is over
-    for (int i = threadIdx.x; i < PATCH; i += kMusclNT) sP[i] = old[i];
+#pragma unroll 8
+    for (int r = 0; r < (PATCH + NT - 1) / NT; ++r) {
+      const int i = tid + r * NT;
+      if ((r + 1) * NT <= PATCH || i < PATCH) sP[i] = old[i];
+    }
     __syncthreads();
-    // evolve the half time step (MH:77-261)
-    for (int j = threadIdx.x; j < NC; j += kMusclNT) {
-      int z, y, x, sheet = -1;
-      if (j < L3) {
-        z = G + j / (L * L);
-        y = G + (j / L) % L;
-        x = G + j % L;
-      } else {
-        const int k = j - L3;
-        sheet = k / (L * L);
-        const int r = k % (L * L), fa = G + r / L, fb = G + r % L;
-        const int gc = (sheet & 1) ? G + L : G - 1;
-        if ((sheet >> 1) == 0) {
-          z = fa;
-          y = fb;
-          x = gc;
-        } else if ((sheet >> 1) == 1) {
-          z = fa;
-          x = fb;
-          y = gc;
-        } else {
-          y = fa;
-          x = fb;
-          z = gc;
-        }
-      }
-      const int p0 = (z * S + y) * S + x;
-      double u[V], slope[3][V], Qt[V];
-#pragma unroll
-      for (int v = 0; v < V; ++v) u[v] = sP[p0 * V + v];
+    // cell (x, y, z), from the interior's first one
+    auto patch_index = [](int x, int y, int z) __device__ { return (((z + G) * S + (y + G)) * S + (x + G)) * V; };
+    // The cell at p0 evolved by half a time step (MH:77-261), and its states at
+    // its faces below and above in direction d: wL and wR (+= dt/2 Qt), or the
+    // cell value itself for the first-order scheme.
+    double Qt[V], slope[3][V];
+    auto evolve = [&](const int p0) __device__ __attribute__((always_inline)) {
       if constexpr (!GODUNOV) {
-        const int step[3] = {1, S, S * S};
+        double u[V];
 #pragma unroll
-        for (int d = 0; d < 3; ++d)
-#pragma unroll
-          for (int v = 0; v < V; ++v)
-            slope[d][v] = minmod(sP[(p0 + step[d]) * V + v] - u[v], u[v] - sP[(p0 - step[d]) * V + v]) * ih[d];
-#pragma unroll
-        for (int v = 0; v < V; ++v) Qt[v] = 0.0;
+        for (int v = 0; v < V; ++v) {
+          u[v] = sP[p0 + v];
+          Qt[v] = 0.0;
+        }
 #pragma unroll
         for (int d = 0; d < 3; ++d) {
           double w[V], F[V];
 #pragma unroll
-          for (int v = 0; v < V; ++v) w[v] = u[v] - 0.5 * h[d] * slope[d][v];
+          for (int v = 0; v < V; ++v)
+            slope[d][v] = minmod(sP[p0 + step[d] * V + v] - u[v], u[v] - sP[p0 - step[d] * V + v]) * ih[d];
+#pragma unroll
+          for (int v = 0; v < V; ++v) w[v] = u[v] - hh[d] * slope[d][v];
           euler_flux_dir(w, d, F);
 #pragma unroll
           for (int v = 0; v < V; ++v) Qt[v] += F[v] * ih[d];
 #pragma unroll
-          for (int v = 0; v < V; ++v) w[v] = u[v] + 0.5 * h[d] * slope[d][v];
+          for (int v = 0; v < V; ++v) w[v] = u[v] + hh[d] * slope[d][v];
           euler_flux_dir(w, d, F);
 #pragma unroll
           for (int v = 0; v < V; ++v) Qt[v] -= F[v] * ih[d];
+          __builtin_amdgcn_sched_barrier(0);  // one direction's temporaries at a time
         }
       }
-      // face states into the face table: the evolved wL/wR (+= dt/2 Qt), or
-      // the cell value itself for the first-order scheme
-      auto face_state = [&](int d, int v, double sign) -> double {
-        if constexpr (GODUNOV) return u[v];
-        return (u[v] + sign * 0.5 * h[d] * slope[d][v]) + 0.5 * dt * Qt[v];
-      };
-      const int co[3] = {x - G, y - G, z - G};
+    };
+    auto below = [&](double u, int d, int v) __device__ {
+      return GODUNOV ? u : (u - hh[d] * slope[d][v]) + hdt * Qt[v];
+    };
+    auto above = [&](double u, int d, int v) __device__ {
+      return GODUNOV ? u : (u + hh[d] * slope[d][v]) + hdt * Qt[v];
+    };
+    // the first ghost layers, sheet 2 d below and 2 d + 1 above the interior in
+    // direction d, by the last wavefronts, which have fewer interior cells
+    if (NT - 1 - tid < 6 * L2) {
+      const int k = NT - 1 - tid, sheet = k / L2, r = k % L2, dir = sheet >> 1;
+      const int gc = (sheet & 1) ? L : -1, ra = r / L, rb = r % L;
+      const int x = dir == 0 ? gc : rb, y = dir == 1 ? gc : (dir == 0 ? rb : ra), z = dir == 2 ? gc : ra;
+      const int p0 = patch_index(x, y, z);
+      evolve(p0);
 #pragma unroll
-      for (int d = 0; d < 3; ++d) {
-        const int fa = (d == 2) ? co[1] : co[2];  // x,y faces: a = z; z faces: a = y
-        const int fb = (d == 0) ? co[1] : co[0];  // x faces: b = y; y,z faces: b = x
-        const bool needL = (sheet < 0) || (sheet == 2 * d + 1);  // wL feeds the face on its left
-        const bool needR = (sheet < 0) || (sheet == 2 * d);      // wR feeds the face on its right
-        if (needL) {
+      for (int v = 0; v < V; ++v) {
+        const double u = sP[p0 + v];
+        double w = 0.0;
 #pragma unroll
-          for (int v = 0; v < V; ++v) sF[fidx(d, 1, v, fa, fb, co[d])] = face_state(d, v, -1.0);
+        for (int d = 0; d < 3; ++d) {  // no run-time index into the registers
+          if (sheet == 2 * d) w = above(u, d, v);
+          if (sheet == 2 * d + 1) w = below(u, d, v);
         }
-        if (needR) {
+        sG[v * 6 * L2 + k] = w;
+      }
+    }
+    if (tid < L3) evolve(patch_index(tid % L, (tid / L) % L, tid / L2));
+    __syncthreads();
+    double q[V];
 #pragma unroll
-          for (int v = 0; v < V; ++v) sF[fidx(d, 0, v, fa, fb, co[d] + 1)] = face_state(d, v, 1.0);
+    for (int d = 0; d < 3; ++d) {
+      // One face per thread: the one below an interior cell, or for the threads
+      // from L^3 on the topmost ones; r numbers the lines along d.
+      asm volatile("" : "+v"(tid));
+      const bool inner = tid < L3;
+      const int x = tid % L, y = (tid / L) % L, z = tid / L2, p0 = patch_index(x, y, z);
+      const int fstep = d == 0 ? 1 : (d == 1 ? L : L2);
+      const int EX = d == 0 ? L + 1 : L, EY = d == 1 ? L + 1 : L;
+      const int r = inner ? (d == 0 ? tid / L : (d == 1 ? z * L + x : tid % L2)) : tid - L3;
+      const int ra = r / L, rb = r % L;
+      const int f0 = inner ? (z * EY + y) * EX + x
+                           : (d == 0 ? r * EX + L : (d == 1 ? (ra * EY + L) * EX + rb : (L * EY + ra) * EX + rb));
+      const bool face = tid < NF;
+      double qL[V], qR[V];
+      if (inner) {
+#pragma unroll
+        for (int v = 0; v < V; ++v) {
+          const double u = sP[p0 + v];
+          qR[v] = below(u, d, v);
+          sX[v * NF + f0 + fstep] = above(u, d, v);
+        }
+      } else if (face) {
+#pragma unroll
+        for (int v = 0; v < V; ++v) {
+          qR[v] = sG[(v * 6 + 2 * d + 1) * L2 + r];
+          sX[v * NF + f0 - L * fstep] = sG[(v * 6 + 2 * d) * L2 + r];
         }
       }
+      __syncthreads();
+      // Rusanov (RUS:98-156), the flux over the left state
+      if (face) {
+        double FL[V], FR[V];
+#pragma unroll
+        for (int v = 0; v < V; ++v) qL[v] = sX[v * NF + f0];
+        const double smax = dmax(Euler<0>::max_abs_eigenvalue(qR, d), Euler<0>::max_abs_eigenvalue(qL, d));
+        if constexpr (DT_MAX) {
+          const double dta = (GODUNOV ? 0.9 : 0.99) / 3 * h[d] / smax;
+          dt_allowed = dta < dt_allowed ? dta : dt_allowed;
+        }
+        euler_flux_dir(qL, d, FL);
+        euler_flux_dir(qR, d, FR);
+#pragma unroll
+        for (int v = 0; v < V; ++v) {
+          double fn = 0.5 * smax * (qL[v] - qR[v]);
+          fn += 0.5 * (FL[v] + FR[v]);
+          sX[v * NF + f0] = fn;
+        }
+      }
+      __syncthreads();
+      // flux differences in the reference's accumulation order (MH:267-329)
+      if (inner) {
+#pragma unroll
+        for (int v = 0; v < V; ++v) {
+          if (d == 0) q[v] = sP[p0 + v];
+          q[v] += cdt[d] * sX[v * NF + f0];
+          q[v] -= cdt[d] * sX[v * NF + f0 + fstep];
+        }
+      }
+      if (d < 2) __syncthreads();  // the next direction rewrites sX
+    }
+    const bool inner = tid < L3;
+    // new values into the other buffer, projection to DG (LIM:69-112) and the
+    // interior min/max (LIM:167-205); every read of sP is before the last
+    // direction's barriers
+#pragma unroll
+    for (int v = 0; v < V; ++v) {
+      const double lo = wave_min(inner ? dmin(DBL_MAX, q[v]) : DBL_MAX);
+      const double hi = -wave_min(inner ? -dmax(-DBL_MAX, q[v]) : DBL_MAX);
+      if (tid % kWave == 0) {
+        red[v * NW + tid / kWave] = lo;
+        red[(V + v) * NW + tid / kWave] = hi;
+      }
+      if (inner) sP[v * L3 + tid] = q[v];
+      __builtin_amdgcn_sched_barrier(0);
     }
     __syncthreads();
-    // Rusanov on every face (RUS:98-156), flux stored over the left state;
-    // dt_max_allowed = min over faces of cflFactor/3 h_d / s_max (MH:267-329)
-    double dt_allowed = DBL_MAX;
-    for (int j = threadIdx.x; j < 3 * NF; j += kMusclNT) {
-      const int d = j / NF, r = j % NF;
-      const int fa = r / (L * (L + 1)), fb = (r / (L + 1)) % L, f = r % (L + 1);
-      double qL[V], qR[V], FL[V], FR[V];
 #pragma unroll
-      for (int v = 0; v < V; ++v) {
-        qL[v] = sF[fidx(d, 0, v, fa, fb, f)];
-        qR[v] = sF[fidx(d, 1, v, fa, fb, f)];
-      }
-      const double smax = dmax(Euler<0>::max_abs_eigenvalue(qR, d), Euler<0>::max_abs_eigenvalue(qL, d));
-      const double dta = (GODUNOV ? 0.9 : 0.99) / 3 * h[d] / smax;  // FV solver CFL / MH:29
-      dt_allowed = dta < dt_allowed ? dta : dt_allowed;
-      euler_flux_dir(qL, d, FL);
-      euler_flux_dir(qR, d, FR);
-#pragma unroll
-      for (int v = 0; v < V; ++v) {
-        double fn = 0.5 * smax * (qL[v] - qR[v]);
-        fn += 0.5 * (FL[v] + FR[v]);
-        sF[fidx(d, 0, v, fa, fb, f)] = fn;
+    for (int r = 0; r < (V * L3 + NT - 1) / NT; ++r) {
+      const int i = tid + r * NT;
+      if (i < V * L3) {
+        const int v = i % V, n = i / V;
+        nw[(((n / (L * L) + G) * S + ((n / L) % L + G)) * S + (n % L + G)) * V + v] = sP[v * L3 + n];
       }
     }
-    if (a.fv_dt_max) {
-      const double m = wave_min(dt_allowed);
-      if ((threadIdx.x & (kWave - 1)) == 0) atomic_min_positive(a.fv_dt_max, m);
+    tensor3<L, B, V, NT>(sP, sLim2uh, sP + T1, sP + T2, sP + OUT, tid);
+    double* const luh = a.luh + (size_t)c * Sh::B3 * V;
+    for (int i = tid; i < Sh::B3 * V; i += NT) luh[i] = sP[OUT + (i % V) * Sh::B3 + i / V];
+    if (tid < 2 * V) {
+      double m = red[tid * NW];
+#pragma unroll 1
+      for (int w = 1; w < NW; ++w) m = tid < V ? dmin(m, red[tid * NW + w]) : dmax(m, red[tid * NW + w]);
+      a.limmm[(size_t)c * 2 * V + tid] = m;
     }
-    __syncthreads();
-    // flux differences in the reference's accumulation order (MH:267-329)
-    for (int j = threadIdx.x; j < L3; j += kMusclNT) {
-      const int iz = j / (L * L), iy = (j / L) % L, ix = j % L;
-      const int p0 = ((iz + G) * S + (iy + G)) * S + (ix + G);
-      double q[V];
-#pragma unroll
-      for (int v = 0; v < V; ++v) {
-        q[v] = sP[p0 * V + v];
-        q[v] += cdt[0] * sF[fidx(0, 0, v, iz, iy, ix)];
-        q[v] -= cdt[0] * sF[fidx(0, 0, v, iz, iy, ix + 1)];
-        q[v] += cdt[1] * sF[fidx(1, 0, v, iz, ix, iy)];
-        q[v] -= cdt[1] * sF[fidx(1, 0, v, iz, ix, iy + 1)];
-        q[v] += cdt[2] * sF[fidx(2, 0, v, iy, ix, iz)];
-        q[v] -= cdt[2] * sF[fidx(2, 0, v, iy, ix, iz + 1)];
-        nw[p0 * V + v] = q[v];
-        sP[p0 * V + v] = q[v];
-      }
-    }
-    __syncthreads();
-    // projection to DG and the patch min/max (sF is free now)
-    double mn[V], mx[V];
-    fv_to_dg<N, kMusclNT>(sP, a.luh + (size_t)c * Sh::B3 * V, sF, sF + L3 * V, sF + 2 * L3 * V, sF + 3 * L3 * V,
-                          sLim2uh, red, mn, mx);
-    if (threadIdx.x == 0) {
-#pragma unroll
-      for (int v = 0; v < V; ++v) {
-        a.limmm[(size_t)c * 2 * V + v] = mn[v];
-        a.limmm[(size_t)c * 2 * V + V + v] = mx[v];
-      }
-      a.cur[c] = (uint8_t)(ob ^ 1);
-    }
+    if (tid == 0) a.cur[c] = (uint8_t)(ob ^ 1);
+    __syncthreads();  // the next patch rewrites sP
+  }
+  if constexpr (DT_MAX) {
+    const double m = wave_min(dt_allowed);
+    if ((threadIdx.x & (kWave - 1)) == 0) atomic_min_positive(a.fv_dt_max, m);
   }
 }
 
@@ -1380,12 +1442,10 @@ hipError_t launch_lim_ghosts(const SolverDesc& sd, const LimArgs& a, bool only_i
 
 hipError_t launch_lim_fv_update(const SolverDesc& sd, const LimArgs& a, bool only_if_irregular, hipStream_t s) {
   return dispatch_lim(sd.order, [&]<int N>() -> hipError_t {
-    if (a.fv_godunov)
-      hipLaunchKernelGGL((lim_fv_update_kernel<N, true>), dim3(persistent_grid(a.ncells)), dim3(kMusclNT), 0, s, a,
-                         only_if_irregular ? 1 : 0);
-    else
-      hipLaunchKernelGGL((lim_fv_update_kernel<N, false>), dim3(persistent_grid(a.ncells)), dim3(kMusclNT), 0, s, a,
-                         only_if_irregular ? 1 : 0);
+    const dim3 grid(persistent_grid(a.ncells, MusclShape<N>::kPerCu)), block(MusclShape<N>::NT);
+    const auto kernel = a.fv_dt_max ? (a.fv_godunov ? lim_fv_update_kernel<N, true, true> : lim_fv_update_kernel<N, false, true>)
+                                    : (a.fv_godunov ? lim_fv_update_kernel<N, true, false> : lim_fv_update_kernel<N, false, false>);
+    hipLaunchKernelGGL(kernel, grid, block, 0, s, a, only_if_irregular ? 1 : 0);
     return hipGetLastError();
   });
 }

@@ -226,3 +226,32 @@ def test_limiting_grid_vs_oracle_mid_size(exa, oracle):
     print(f"  FV-active {(st >= 2).mean():.3f}, irregular steps {irr_prev}", flush=True)
     assert irr_prev > 0 and (st >= 2).any()
     g.close()
+
+
+@pytest.mark.parametrize("godunov", [False, True])
+@pytest.mark.parametrize("order,n", [(2, 14), (3, 13)])
+def test_more_patches_than_resident_workgroups_vs_oracle(exa, oracle, order, n, godunov):
+    """The patch kernel's workgroups are persistent: more FV-active cells than
+    workgroups on the device (2 per compute unit at N=3, 3 at N=2), so that one
+    takes several patches in turn.  Bars of the grids above."""
+    print(f"case: many patches, N={order} {n}^3 godunov={godunov}", flush=True)
+    steps = 3
+    nodes = np.array([oracle.table(oracle.T_NODES, order, i) for i in range(order + 1)])
+    luh = blast_cells(order, n, nodes=nodes, radius=0.3)
+    lim_ic = blast_cells(order, n, subcells=True, radius=0.3)
+    g = exa.LimitingGrid(exa.euler_solver(order), n, boundary=exa.BC_TRANSMISSIVE,
+                         fv_scheme=exa.FV_GODUNOV if godunov else exa.FV_MUSCLHANCOCK)
+    g.upload(luh, lim_ic)
+    o = oracle.LimitingGrid(oracle.make_solver(order), n, periodic=False,
+                            fv_scheme=oracle.FV_GODUNOV if godunov else oracle.FV_MUSCLHANCOCK)
+    o.set_solution(luh, lim_ic)
+    g.step(steps)
+    ost, _, _ = o.step(steps)
+    st, _ = g.status()
+    print(f"  FV-active cells {(st >= 2).sum()}", flush=True)
+    assert (st >= 2).sum() > 800
+    assert np.array_equal(st, ost[-1])
+    sol, osol = g.solution().reshape(-1, 5), o.solution().reshape(-1, 5)
+    for v in range(5):
+        assert rel_max(sol[:, v], osol[:, v]) <= 1e-11, v
+    g.close()
