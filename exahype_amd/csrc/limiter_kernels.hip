@@ -621,14 +621,16 @@ __device__ inline void tensor3_rows(const double* in, double* t1, double* t2, in
 constexpr int kStatusCells = 4;  // cells (wavefronts) per workgroup of the status kernel
 
 template <int N>
-// Registers capped for five wavefronts per SIMD (109 -> at most 102 VGPRs,
-// no scratch; 2.83 -> 2.73 ms at 81^3 N=3), six spill.
+// Registers capped for five wavefronts per SIMD (88 used at N=3); six spill.
+// FP64 issue and LDS both near their limits: 208,000 cells at N=3 1.02 -> 0.87
+// ms with the minima reduced by register moves, one instruction per minimum and
+// the extrema kept in LDS instead of selected into registers.
 __global__ __launch_bounds__(kStatusCells * kWave, 5) void lim_update_status_kernel(LimArgs a) {
   using Sh = LimShape<N>;
   constexpr int B = Sh::B, B2 = B * B, B3 = Sh::B3, L = Sh::L, L3 = Sh::L3, V = Sh::V, PATCH = Sh::PATCH;
   static_assert(B3 <= kWave, "one node per lane");
   constexpr int T1 = B * B * L, T2 = B * L * L;  // the subcell transform's; the Lobatto one's are smaller
-  constexpr int PER = V * B3 + T1 + T2 + 12 * V;  // sQ, t1, t2, face extrema
+  constexpr int PER = V * B3 + T1 + T2 + 14 * V;  // sQ, t1, t2, face extrema, local extrema
   __shared__ double sWave[kStatusCells * PER];
   // no workgroup barrier: each wavefront works in its own part of sWave
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave;
@@ -638,6 +640,7 @@ __global__ __launch_bounds__(kStatusCells * kWave, 5) void lim_update_status_ker
   double* const t1 = sQ + V * B3;
   double* const t2 = t1 + T1;
   double* const sBnd = t2 + T2;
+  double* const sMM = sBnd + 12 * V;
   // loads whose latency the DG update hides: the merged face extrema (one
   // lane per face-block entry) and the neighbours' previous statuses (one
   // lane per face)
@@ -717,37 +720,25 @@ __global__ __launch_bounds__(kStatusCells * kWave, 5) void lim_update_status_ker
   }
   wave_lds_sync();
   // local min/max (LIM:210-368): Gauss-Legendre nodes, Lobatto nodes,
-  // subcell means, one variable at a time
-  double mn[V], mx[V];
+  // subcell means, one variable at a time (fmin and fmax are one instruction,
+  // and the same as a < b ? a : b where the left value is never a NaN)
 #pragma unroll 1
   for (int v = 0; v < V; ++v) {
     double lo = DBL_MAX, hi = -DBL_MAX;
     if (active) {  // B3 <= kWave: one node per lane
-      lo = dmin(lo, sQ[v * B3 + lane]);
-      hi = dmax(hi, sQ[v * B3 + lane]);
+      lo = fmin(lo, sQ[v * B3 + lane]);
+      hi = fmax(hi, sQ[v * B3 + lane]);
     }
     auto fold = [&](int, int, double u) {
-      lo = dmin(lo, u);
-      hi = dmax(hi, u);
+      lo = fmin(lo, u);
+      hi = fmax(hi, u);
     };
     tensor3_rows<N, kTabUh2Lob, B, B>(sQ + v * B3, t1, t2, lane, fold);  // Lobatto nodes
     tensor3_rows<N, kTabUh2Lim, B, L>(sQ + v * B3, t1, t2, lane, fold);  // subcell means
     lo = wave_min(lo);
     hi = -wave_min(-hi);
-    // a register array indexed by the rolled v would live in scratch memory:
-    // select into the unrolled slots instead
-#pragma unroll
-    for (int w = 0; w < V; ++w) {
-      mn[w] = (w == v) ? lo : mn[w];
-      mx[w] = (w == v) ? hi : mx[w];
-    }
-  }
-  if (lane == 0) {
-#pragma unroll
-    for (int v = 0; v < V; ++v) {
-      a.loc_mm[(size_t)c * 2 * V + v] = mn[v];
-      a.loc_mm[(size_t)c * 2 * V + V + v] = mx[v];
-    }
+    sMM[v] = lo;  // every lane the same
+    sMM[V + v] = hi;
   }
   // DMP (LIM:114-165) against the merged boundary extrema, staged in LDS
   double* bmn = a.mn + (size_t)c * 6 * V;
@@ -756,15 +747,21 @@ __global__ __launch_bounds__(kStatusCells * kWave, 5) void lim_update_status_ker
   if (lane < 6 * V) sSub[lane] = bnd;
   if (lane >= 32 && lane < 32 + 6 * V) sSub[6 * V + lane - 32] = bnd;
   wave_lds_sync();
+  if (lane < 2 * V) a.loc_mm[(size_t)c * 2 * V + lane] = sMM[lane];
   bool ok = true;
-  double bMin[V], bMax[V];
+  double mn[V], mx[V], bMin[V], bMax[V];
+#pragma unroll
+  for (int v = 0; v < V; ++v) {
+    mn[v] = sMM[v];
+    mx[v] = sMM[V + v];
+  }
 #pragma unroll
   for (int v = 0; v < V; ++v) {
     double lo = sSub[v], hi = sSub[6 * V + v];
 #pragma unroll
     for (int f = 1; f < 6; ++f) {
-      lo = dmin(lo, sSub[f * V + v]);
-      hi = dmax(hi, sSub[6 * V + f * V + v]);
+      lo = fmin(lo, sSub[f * V + v]);
+      hi = fmax(hi, sSub[6 * V + f * V + v]);
     }
     double sd = (hi - lo) * a.scaling;
     sd = dmax(sd, a.relax);

