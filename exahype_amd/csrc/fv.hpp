@@ -80,8 +80,8 @@ hipError_t launch_fv_euler_ic(const ICArgs& ic, double* planes, int X, int Y, in
                               hipStream_t s);
 
 // Workgroup shape of the update kernel: kFvRows wavefronts, each a row of 64
-// consecutive subcells along x; rows 1..kFvRows-2 and lanes 1..62 produce
-// output, the outer rows and lanes supply neighbour values.
+// consecutive subcells along x; every row and lanes 1..62 produce output, the
+// outer lanes supply neighbour values.
 constexpr int kFvRows = 8;
 constexpr int kFvOutX = 64 - 2;
 

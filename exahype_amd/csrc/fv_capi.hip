@@ -100,23 +100,27 @@ void fv_free(exa_fvgrid* g) {
   delete g;
 }
 
-// Tiling of the update kernel: 62 x 6 columns per workgroup, the z range cut
-// into chunks so that the launch has about 8 workgroups per CU in total,
-// chunks of at least 16 planes.
+// Tiling of the update kernel: 62 x 8 columns per workgroup, the z range cut
+// into chunks.  The cut is the one with the shortest run: the rounds that the
+// workgroups take over the device (two resident per CU, the tiles dealt to
+// eight XCDs) times the planes of a chunk and two more for its first face.
 void fv_tiling(exa_fvgrid* g) {
   int dev = 0, cus = 256;
   if (hipGetDevice(&dev) == hipSuccess) (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
   exa::FvGridArgs& a = g->args;
-  constexpr int out_rows = exa::kFvRows - 2;
   a.nsx = (g->X + exa::kFvOutX - 1) / exa::kFvOutX;
-  a.nry = (g->Y + out_rows - 1) / out_rows;
-  const long per_chunk = (long)a.nsx * a.nry;
-  long nzc = (8L * cus + per_chunk - 1) / per_chunk;
-  const long max_chunks = g->Z / 16 > 1 ? g->Z / 16 : 1;
-  if (nzc > max_chunks) nzc = max_chunks;
-  if (nzc < 1) nzc = 1;
-  a.zlen = (int)((g->Z + nzc - 1) / nzc);
-  a.nzc = (g->Z + a.zlen - 1) / a.zlen;
+  a.nry = (g->Y + exa::kFvRows - 1) / exa::kFvRows;
+  const long per_chunk = (long)a.nsx * a.nry, slots = cus / 8 > 0 ? 2 * (cus / 8) : 2;  // of one XCD
+  long best = 0;
+  for (int nzc = 1; nzc == 1 || nzc <= g->Z / 4; ++nzc) {
+    const int zlen = (g->Z + nzc - 1) / nzc, chunks = (g->Z + zlen - 1) / zlen;
+    const long rounds = ((per_chunk * chunks + 7) / 8 + slots - 1) / slots, cost = rounds * (zlen + 2);
+    if (best == 0 || cost < best) {
+      best = cost;
+      a.zlen = zlen;
+      a.nzc = chunks;
+    }
+  }
   a.ntiles = (int)(per_chunk * a.nzc);
 }
 

@@ -18,6 +18,7 @@
 #include <cfloat>
 #include <cmath>
 
+#include "line_ops.hpp"
 #include "exa_device.hpp"
 #include "fv.hpp"
 #include "fv_device.hpp"
@@ -43,14 +44,10 @@ __device__ inline CellBase cell_base(const double* q) {
   return b;
 }
 
-// Largest |eigenvalue| in direction d: max_element of |(u-c, u, u, u, u+c)|.
+// Largest |eigenvalue| in direction d: max_element of |(u-c, u, u, u, u+c)|,
+// which is |u| + c to the last bit, c >= 0 (and a NaN where c is one).
 __device__ inline double cell_lambda(const double* q, const CellBase& b, int d) {
-  const double u_n = q[d + 1] * b.irho;
-  const double l0 = fabs(u_n - b.cs), l1 = fabs(u_n), l4 = fabs(u_n + b.cs);
-  double m = l0;
-  m = (m < l1) ? l1 : m;
-  m = (m < l4) ? l4 : m;
-  return m;
+  return fabs(q[d + 1] * b.irho) + b.cs;
 }
 
 __device__ inline void cell_flux(const double* q, const CellBase& b, int d, double* F) {
@@ -149,26 +146,32 @@ __global__ __launch_bounds__(256) void godunov_patch_kernel(GodunovPatchArgs a) 
 }
 
 // ---------------------------------------------------------------------------
-// Grid update.  A workgroup owns a tile of 62 x 6 subcell columns and
-// walks a range of z planes.  Wavefront w holds row y0 - 1 + w, lane l
-// column x0 - 1 + l, so the outer rows and lanes carry the neighbours of the
-// tile.  Per plane and column the subcell's pressure and sound speed are
-// formed once, each face flux once:
+// Grid update.  A workgroup owns a tile of 62 x 8 subcell columns and walks a
+// range of z planes.  Wavefront w holds row y0 + w, lane l column x0 - 1 + l,
+// so the outer lanes carry the neighbours of the tile.  Per plane and column
+// the subcell's pressure and sound speed are formed once, x and z faces once:
 //   x faces: lane l forms the face to its right from lane l+1's state,
 //            directional flux and eigenvalue (DPP lane shifts), and passes
 //            it to lane l+1 as that lane's left face;
-//   y faces: rows exchange state, y flux and eigenvalue through LDS; row w
-//            forms the face above it and leaves it in LDS for row w+1;
 //   z faces: carried along the walk (the face above plane z is the face
-//            below plane z+1).
+//            below plane z+1);
+//   y faces: rows exchange their states through LDS, and both rows of a face
+//            form it: 50 instructions more, but one barrier per plane (two
+//            planes' states in LDS) instead of two.  The first and the last
+//            wavefront also supply the row beyond the tile.
 // The update is followed by the new subcell's eigenvalue maxima for the next
 // stable dt (startNewTimeStep, FVS:553-574), reduced over the wavefront and
 // into state->lam_max.  Reads per step: each subcell once from the tile, plus
-// the tile borders (1/31 along x, 1/3 along y, read again by the
-// neighbouring tile, partly from L2); writes: each subcell once.  Eight
-// wavefronts per workgroup and two workgroups per CU (114 VGPRs, 64 KiB of
-// LDS each) measured faster than one workgroup of sixteen, whose barriers
-// hold all sixteen wavefronts of the CU.
+// the tile borders (1/31 along x, 1/4 along y, read again by the neighbouring
+// tile, mostly from L2); writes: each subcell once.
+//
+// Bound by the latency of a plane (divide, square root and exchange in a row)
+// with four wavefronts per SIMD, which is what 126 registers and 80 KB of LDS
+// a workgroup allow.  270^3 subcells: 0.635 -> 0.439 ms a step, 2.5 -> 3.6 TB/s
+// of the 80 bytes a subcell has to move: 5% by the single barrier and the
+// eigenvalue as |u| + c, 19% by all eight rows producing output (six of eight
+// did) and the z chunks cut for whole rounds of workgroups, 10% by one atomic
+// per workgroup and direction instead of one per wavefront.
 // ---------------------------------------------------------------------------
 __device__ inline int wrap_index(int i, int n, int periodic) {
   if (periodic) {
@@ -200,16 +203,31 @@ __device__ inline void atomic_max_positive(unsigned long long* slot, double v) {
   asm volatile("" : : "v"(old));
 }
 
-// Wavefront maximum of one direction's eigenvalue maxima into the state.
-__device__ inline void reduce_lambda(FvState* st, int d, double lm) {
-  const double m = -wave_min(-lm);
-  if ((threadIdx.x & (kWave - 1)) == 0 && m > 0.0) atomic_max_positive(&st->lam_max[d], m);
+// The workgroup's eigenvalue maxima per direction into the state.  Atomics on
+// one address take 12 ns each whichever CU they come from, so a workgroup sends
+// one per direction, and none where the state already holds as much (a stale
+// value read here only costs the atomic): with one per wavefront they were the
+// longest part of a step on small grids (60x90x200 subcells 129 -> 62 us a step
+// with the tiles below) and of the stand-alone reductions (20 million subcells
+// 1.15 -> 0.18 ms).
+template <int NT>
+__device__ inline void reduce_lambda(FvState* st, double lmx, double lmy, double lmz, double* red) {
+  constexpr int NW = NT / kWave;  // red: 3 NW doubles of LDS
+  const double m[3] = {-wave_min(-lmx), -wave_min(-lmy), -wave_min(-lmz)};
+#pragma unroll
+  for (int d = 0; d < 3; ++d) red[d * NW + threadIdx.x / kWave] = m[d];  // every lane of the wavefront the same
+  __syncthreads();
+  if (threadIdx.x >= 3) return;
+  const int d = threadIdx.x;
+  double best = red[d * NW];
+  for (int w = 1; w < NW; ++w) best = fmax(best, red[d * NW + w]);
+  const unsigned long long held = __hip_atomic_load(&st->lam_max[d], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (best > __longlong_as_double((long long)held)) atomic_max_positive(&st->lam_max[d], best);
 }
 
-__global__ __launch_bounds__(kWave * kFvRows) void fv_godunov_kernel(FvGridArgs a) {
-  constexpr int ROWS = kFvRows, OUT_ROWS = ROWS - 2;
-  __shared__ double sQ[ROWS][11][kWave];  // state (5), y flux (5), y eigenvalue
-  __shared__ double sFy[ROWS][5][kWave];  // face above the row
+__global__ __launch_bounds__(kWave * kFvRows, 4) void fv_godunov_kernel(FvGridArgs a) {
+  constexpr int ROWS = kFvRows;
+  __shared__ double sQ[2][ROWS + 2][8][kWave];  // even and odd planes: state (5), 1/rho, p, c
   // XCD-aware tile order: workgroup b runs on XCD b % 8; give each XCD a
   // contiguous run of tiles with the x strip fastest, so that the tiles that
   // share border columns (x neighbours, adjacent in the run) and border rows
@@ -220,17 +238,20 @@ __global__ __launch_bounds__(kWave * kFvRows) void fv_godunov_kernel(FvGridArgs 
   if (t >= a.ntiles) return;  // the whole workgroup
   const int sx = t % a.nsx, r2 = t / a.nsx, ry = r2 % a.nry, cz = r2 / a.nry;
   const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
-  const int xp = sx * kFvOutX - 1 + lane, yp = ry * OUT_ROWS - 1 + w;
+  const int xp = sx * kFvOutX - 1 + lane, yp = ry * ROWS + w;
   const int xs = wrap_index(xp, a.X, a.periodic), ys = wrap_index(yp, a.Y, a.periodic);
-  const bool out_row = w >= 1 && w <= OUT_ROWS && yp < a.Y;  // uniform per wavefront
+  const bool out_row = yp < a.Y;  // uniform per wavefront
   const bool out = out_row && lane >= 1 && lane <= kFvOutX && xp < a.X;
-  const bool face_above = out_row || w == 0;
   const size_t plane = (size_t)a.X * a.Y, vol = plane * (size_t)a.Z;
   const size_t col = (size_t)ys * a.X + xs;
+  // the first and the last row's wavefronts also supply the row beyond
+  const bool edge = w == 0 || w == ROWS - 1;
+  const int slot = w == 0 ? 0 : ROWS + 1;
+  const size_t edge_col = (size_t)wrap_index(w == 0 ? yp - 1 : yp + 1, a.Y, a.periodic) * a.X + xs;
   const int z0 = cz * a.zlen, z1 = min(a.Z, z0 + a.zlen);
   const double dt = a.state->dt;
-  const double cdt[3] = {dt / a.h[0], dt / a.h[1], dt / a.h[2]};
-  auto load = [&](int z, double* q) __device__ {
+  const double cdt[3] = {wave_uniform(dt / a.h[0]), wave_uniform(dt / a.h[1]), wave_uniform(dt / a.h[2])};
+  auto load = [&](int z, size_t col, double* q) __device__ {
     const size_t o = (size_t)wrap_index(z, a.Z, a.periodic) * plane + col;
 #pragma unroll
     for (int v = 0; v < 5; ++v) q[v] = a.u[v * vol + o];
@@ -238,13 +259,14 @@ __global__ __launch_bounds__(kWave * kFvRows) void fv_godunov_kernel(FvGridArgs 
 
   // every row walks with the next plane's state already loaded and the one
   // after in flight (the rows without output only supply their state)
-  double q[5], qn[5], qnn[5], fzlo[5];
+  double q[5], qn[5], qnn[5], qe[5], fzlo[5];
   CellBase b{};
-  load(z0, q);
-  load(z0 + 1, qn);
+  load(z0, col, q);
+  load(z0 + 1, col, qn);
+  if (edge) load(z0, edge_col, qe);
   if (out_row) {
     double qm[5], Fm[5], Fz[5];
-    load(z0 - 1, qm);
+    load(z0 - 1, col, qm);
     const CellBase bm = cell_base(qm);
     b = cell_base(q);
     cell_flux(qm, bm, 2, Fm);
@@ -253,34 +275,24 @@ __global__ __launch_bounds__(kWave * kFvRows) void fv_godunov_kernel(FvGridArgs 
   }
   double lmx = 0.0, lmy = 0.0, lmz = 0.0;
   for (int z = z0; z < z1; ++z) {
-    // phase A: this row's state, y flux and y eigenvalue into LDS
-    load(z + 2, qnn);  // in flight during this plane
+    double(*const sZ)[8][kWave] = sQ[(z - z0) & 1];
+    auto supply = [&](int r, const double* s, const CellBase& bs) __device__ {
+#pragma unroll
+      for (int v = 0; v < 5; ++v) sZ[r][v][lane] = s[v];
+      sZ[r][5][lane] = bs.irho;
+      sZ[r][6][lane] = bs.p;
+      sZ[r][7][lane] = bs.cs;
+    };
+    if (edge) {
+      supply(slot, qe, cell_base(qe));
+      load(z + 1, edge_col, qe);
+    }
+    load(z + 2, col, qnn);  // in flight during this plane
     if (!out_row) b = cell_base(q);
-    {
-      double Fy[5];
-      cell_flux(q, b, 1, Fy);
-#pragma unroll
-      for (int v = 0; v < 5; ++v) {
-        sQ[w][v][lane] = q[v];
-        sQ[w][5 + v][lane] = Fy[v];
-      }
-      sQ[w][10][lane] = cell_lambda(q, b, 1);
-    }
-    __syncthreads();
-    // phase B: the y face above the row into LDS; the x faces
-    if (face_above) {
-      double Fy[5], qa[5], Fa[5], fyhi[5];
-      cell_flux(q, b, 1, Fy);
-#pragma unroll
-      for (int v = 0; v < 5; ++v) {
-        qa[v] = sQ[w + 1][v][lane];
-        Fa[v] = sQ[w + 1][5 + v][lane];
-      }
-      rusanov_from_parts(q, Fy, cell_lambda(q, b, 1), qa, Fa, sQ[w + 1][10][lane], fyhi);
-#pragma unroll
-      for (int v = 0; v < 5; ++v) sFy[w][v][lane] = fyhi[v];
-    }
-    double un[5];
+    supply(w + 1, q, b);
+    // what needs no other row before the plane's barrier: x faces, z face above
+    double un[5], fzhi[5];
+    CellBase bn{};
     if (out_row) {
       double Fx[5], qr[5], Fr[5], fxhi[5];
       cell_flux(q, b, 0, Fx);
@@ -298,33 +310,51 @@ __global__ __launch_bounds__(kWave * kFvRows) void fv_godunov_kernel(FvGridArgs 
         un[v] += cdt[0] * fxlo;
         un[v] -= cdt[0] * fxhi[v];
       }
-    }
-    __syncthreads();
-    // phase C: y and z terms, store, eigenvalue maxima of the new state
-    if (out_row) {
-#pragma unroll
-      for (int v = 0; v < 5; ++v) {
-        un[v] += cdt[1] * sFy[w - 1][v][lane];
-        un[v] -= cdt[1] * sFy[w][v][lane];
-      }
-      const CellBase bn = cell_base(qn);
-      double Fz[5], Fzn[5], fzhi[5];
+      bn = cell_base(qn);
+      double Fz[5], Fzn[5];
       cell_flux(q, b, 2, Fz);
       cell_flux(qn, bn, 2, Fzn);
       rusanov_from_parts(q, Fz, cell_lambda(q, b, 2), qn, Fzn, cell_lambda(qn, bn, 2), fzhi);
+    }
+    __syncthreads();
+    // both y faces (each is formed by both its rows: no second barrier), z
+    // terms, store, eigenvalue maxima of the new state
+    if (out_row) {
+      double Fy[5], qa[5], Fa[5], fy[5];
+      CellBase ba;
+      auto row = [&](int r) __device__ {
+#pragma unroll
+        for (int v = 0; v < 5; ++v) qa[v] = sZ[r][v][lane];
+        ba = {sZ[r][5][lane], sZ[r][6][lane], sZ[r][7][lane]};
+        cell_flux(qa, ba, 1, Fa);
+      };
+      cell_flux(q, b, 1, Fy);
+      const double ly = cell_lambda(q, b, 1);
+      row(w);
+      rusanov_from_parts(qa, Fa, cell_lambda(qa, ba, 1), q, Fy, ly, fy);
+#pragma unroll
+      for (int v = 0; v < 5; ++v) un[v] += cdt[1] * fy[v];
+      __builtin_amdgcn_sched_barrier(0);  // one row's values at a time in registers
+      row(w + 2);
+      rusanov_from_parts(q, Fy, ly, qa, Fa, cell_lambda(qa, ba, 1), fy);
 #pragma unroll
       for (int v = 0; v < 5; ++v) {
+        un[v] -= cdt[1] * fy[v];
         un[v] += cdt[2] * fzlo[v];
         un[v] -= cdt[2] * fzhi[v];
       }
+      // Loads and stores return in order: waited for after the stores, which only
+      // some lanes make, the plane in flight would cost their round trip, too.
+#pragma unroll
+      for (int v = 0; v < 5; ++v) asm volatile("" : "+v"(qnn[v]), "+v"(qe[v]));
       if (out) {
         const size_t o = (size_t)z * plane + col;
 #pragma unroll
         for (int v = 0; v < 5; ++v) a.un[v * vol + o] = un[v];
         const CellBase bu = cell_base(un);
-        lmx = dmax(lmx, cell_lambda(un, bu, 0));
-        lmy = dmax(lmy, cell_lambda(un, bu, 1));
-        lmz = dmax(lmz, cell_lambda(un, bu, 2));
+        lmx = fmax(lmx, cell_lambda(un, bu, 0));
+        lmy = fmax(lmy, cell_lambda(un, bu, 1));
+        lmz = fmax(lmz, cell_lambda(un, bu, 2));
       }
       // walk one plane up
 #pragma unroll
@@ -337,9 +367,8 @@ __global__ __launch_bounds__(kWave * kFvRows) void fv_godunov_kernel(FvGridArgs 
       qn[v] = qnn[v];
     }
   }
-  reduce_lambda(a.state, 0, lmx);
-  reduce_lambda(a.state, 1, lmy);
-  reduce_lambda(a.state, 2, lmz);
+  __syncthreads();  // sQ has been read
+  reduce_lambda<kWave * kFvRows>(a.state, lmx, lmy, lmz, &sQ[0][0][0][0]);
 }
 
 // dt = min over d of ch[d] / lam_max[d] (the minimum over subcells and
@@ -376,9 +405,8 @@ __global__ __launch_bounds__(256) void fv_lambda_kernel(FvGridArgs a) {
     lmy = dmax(lmy, cell_lambda(q, b, 1));
     lmz = dmax(lmz, cell_lambda(q, b, 2));
   }
-  reduce_lambda(a.state, 0, lmx);
-  reduce_lambda(a.state, 1, lmy);
-  reduce_lambda(a.state, 2, lmz);
+  __shared__ double red[3 * 256 / kWave];
+  reduce_lambda<256>(a.state, lmx, lmy, lmz, red);
 }
 
 __global__ void fv_begin_kernel(FvState* st) {
@@ -460,9 +488,8 @@ __global__ __launch_bounds__(256) void fv_patch_lambda_kernel(const double* lim,
 #pragma unroll
     for (int d = 0; d < 3; ++d) lm[d] = dmax(lm[d], cell_lambda(q, b, d));
   }
-  reduce_lambda(st, 0, lm[0]);
-  reduce_lambda(st, 1, lm[1]);
-  reduce_lambda(st, 2, lm[2]);
+  __shared__ double red[3 * 256 / kWave];
+  reduce_lambda<256>(st, lm[0], lm[1], lm[2], red);
 }
 
 // cells [cells][L^3][5] (the reference's patch interiors, cell-major) <->

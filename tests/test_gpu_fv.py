@@ -113,6 +113,28 @@ def test_fvgrid_vs_oracle(exa, oracle, n, L, periodic):
     g.close()
 
 
+@pytest.mark.parametrize("periodic", [True, False])
+@pytest.mark.parametrize("n,L", [((1, 1, 1), 7), ((1, 1, 3), 8), ((7, 1, 1), 9), ((2, 1, 1), 31), ((8, 2, 1), 8),
+                                 ((1, 1, 1), 17)])
+def test_fvgrid_tile_edges_vs_oracle(exa, oracle, n, L, periodic):
+    """The update's tiles of 62 x 8 columns: one row less and more than a tile,
+    whole tiles, a strip of one or two columns, one z chunk and several (bar of
+    the grids above)."""
+    print(f"case: FV grid tile edges, cells {n} L={L} periodic={periodic}", flush=True)
+    _, cells = fv_grid_state(n, L, fv_smooth)
+    g = exa.FVGrid(exa.euler_solver(3), L, n, boundary=exa.BC_PERIODIC if periodic else exa.BC_TRANSMISSIVE)
+    g.upload(cells)
+    o = oracle.FVGrid(oracle.make_solver(3), oracle.FV_GODUNOV, L, n, periodic=periodic)
+    o.set_solution(cells)
+    for k in range(3):
+        g.step(1)
+        o.step(1)
+        err = _var_err(g.solution(), o.solution())
+        assert err <= 1e-12, f"solution after step {k}: {err:.3e}"
+        assert abs(g.time()[1] - o.dt()) <= 1e-13 * o.dt()
+    g.close()
+
+
 def test_fvgrid_init_euler_matches_host(exa):
     print("case: FV grid device initial condition vs host formula, 3x2x2 cells L=6", flush=True)
     n, L = (3, 2, 2), 6
