@@ -46,7 +46,7 @@ struct LimArgs {
   double* mn;         // [cells][6][V] solution minima per face block
   double* mx;         // [cells][6][V]
   double* limmm;      // [cells][2][V] min/max over the FV patch interior
-  int* flags;         // [0] irregular change this step; [1] FV list size; [2] recompute list size
+  int* flags;         // kLimFlags counters, see kLimFlagIrregular
   int* fv_list;       // [cells]
   int* rc_list;       // [cells] cells with status > 0 after an irregular change (rolled back)
   double* loc_mm;     // [cells][2][V] local min/max of the DG solution after the update
@@ -65,12 +65,22 @@ struct LimArgs {
   int fv_godunov;
 };
 
-enum : int { kLimFlagIrregular = 0, kLimFlagFvCount = 1, kLimFlagRcCount = 2 };
+// kLimFlagFvAgain: length of the FV list as the rollback rebuilds it after an
+// irregular change; kLimFlagSteps: steps with one since the start of the run.
+enum : int {
+  kLimFlagIrregular = 0,
+  kLimFlagFvCount = 1,
+  kLimFlagRcCount = 2,
+  kLimFlagSteps = 3,
+  kLimFlagFvAgain = 4,
+  kLimFlags = 5
+};
 
 // The launch_* functions below take the solver order (2..kLimMaxOrder, Euler,
 // FP64).  "all" launches cover every cell; the FV launches walk fv_list.
 bool limiter_supported(const SolverDesc& sd);
-// pst = st; flags cleared; FV list of cells with st >= A.
+// pst = st; flags cleared; FV list of cells with st >= A (its length is zero
+// before: launch_lim_update_status and launch_lim_init leave it so).
 hipError_t launch_lim_begin_step(const SolverDesc& sd, const LimArgs& a, hipStream_t s);
 // per interior face: merge the min/max face blocks (mergeSolutionMinMaxOnFace)
 hipError_t launch_lim_minmax_merge(const SolverDesc& sd, const LimArgs& a, const FaceDesc* faces, long nfaces,

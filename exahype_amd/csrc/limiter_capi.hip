@@ -63,10 +63,6 @@ __global__ __launch_bounds__(256) void blast_kernel(double* out, int nx, int ny,
 }
 #pragma clang fp contract(on)
 
-__global__ void lim_count_irregular_kernel(int* flags) {
-  if (threadIdx.x == 0) flags[3] += flags[exa::kLimFlagIrregular];
-}
-
 }  // namespace
 
 struct exa_lgrid {
@@ -254,10 +250,6 @@ hipError_t lstep(exa_lgrid* g) {
       if (r == hipSuccess) r = exa::launch_lim_ghosts(sd, a, true, s);
       if (r == hipSuccess) r = exa::launch_lim_fv_update(sd, a, true, s);
       if (r == hipSuccess) r = exa::launch_lim_recompute_finish(sd, a, s);
-      if (r == hipSuccess) {
-        hipLaunchKernelGGL(lim_count_irregular_kernel, dim3(1), dim3(64), 0, s, g->flags);
-        r = hipGetLastError();
-      }
       if (r == hipSuccess && g->fused_ts) r = exa::launch_lim_repredict_mask(a, g->st2, s);
       return r;
     });
@@ -340,7 +332,7 @@ extern "C" int exa_lgrid_create(const exa_solver* s, int nx, int ny, int nz, con
   A((void**)&g->st2, sizeof(int) * ncells);
   A((void**)&g->itc, sizeof(int) * ncells);
   A((void**)&g->nbr, sizeof(int) * ncells * 6);
-  A((void**)&g->flags, sizeof(int) * 4);
+  A((void**)&g->flags, sizeof(int) * exa::kLimFlags);
   A((void**)&g->fv_list, sizeof(int) * ncells);
   A((void**)&g->rc_list, sizeof(int) * ncells);
   A((void**)&g->loc_mm, sizeof(double) * ncells * 10);
@@ -353,7 +345,7 @@ extern "C" int exa_lgrid_create(const exa_solver* s, int nx, int ny, int nz, con
   }
   // patch edges and corners must read zero forever (FiniteVolumesSolver.cpp:477-481)
   if (e == hipSuccess) e = hipMemsetAsync(g->lim, 0, sizeof(double) * ncells * 2 * patch, g->stream);
-  if (e == hipSuccess) e = hipMemsetAsync(g->flags, 0, sizeof(int) * 4, g->stream);
+  if (e == hipSuccess) e = hipMemsetAsync(g->flags, 0, sizeof(int) * exa::kLimFlags, g->stream);
   if (e == hipSuccess) e = hipMemcpyAsync(g->d_dx, g->dx, sizeof(double) * 3, hipMemcpyHostToDevice, g->stream);
   // neighbours and the interior face list (each face once, owned by its left cell)
   std::vector<int> nbr(ncells * 6);
@@ -403,7 +395,7 @@ extern "C" long exa_lgrid_num_cells(const exa_lgrid* g) { return g ? g->ncells :
 
 static int lgrid_init_from_device(exa_lgrid* g, const double* d_lim_ic) {
   const exa::LimArgs a = largs(g);
-  EXA_TRY(hipMemsetAsync(g->flags, 0, sizeof(int) * 4, g->stream));  // new run: counters from zero
+  EXA_TRY(hipMemsetAsync(g->flags, 0, sizeof(int) * exa::kLimFlags, g->stream));  // new run: counters from zero
   EXA_TRY(exa::launch_lim_init(g->sd, a, d_lim_ic, g->stream));
   EXA_TRY(lstart(g));
   EXA_TRY(hipStreamSynchronize(g->stream));
@@ -496,11 +488,11 @@ extern "C" int exa_lgrid_download(exa_lgrid* g, double* luh) {
 
 extern "C" int exa_lgrid_status(exa_lgrid* g, int* status, long* irregular_steps) {
   if (!g) return EXA_E_INVALID;
-  int flags[4];
+  int flags[exa::kLimFlags];
   if (status) EXA_TRY(hipMemcpyAsync(status, g->st, sizeof(int) * g->ncells, hipMemcpyDeviceToHost, g->stream));
   EXA_TRY(hipMemcpyAsync(flags, g->flags, sizeof(flags), hipMemcpyDeviceToHost, g->stream));
   EXA_TRY(hipStreamSynchronize(g->stream));
-  if (irregular_steps) *irregular_steps = flags[3];
+  if (irregular_steps) *irregular_steps = flags[exa::kLimFlagSteps];
   return EXA_OK;
 }
 
@@ -664,7 +656,7 @@ extern "C" int exa_musclhancock_solution_update(const exa_solver* s, double* luh
   EXA_TRY(d_mm.alloc(sizeof(double) * 10));
   EXA_TRY(d_cur.alloc(1));
   EXA_TRY(d_list.alloc(sizeof(int)));
-  EXA_TRY(d_flags.alloc(sizeof(int) * 4));
+  EXA_TRY(d_flags.alloc(sizeof(int) * exa::kLimFlags));
   EXA_TRY(d_dx.alloc(sizeof(double) * 3));
   EXA_TRY(d_state.alloc(sizeof(exa::StepState)));
   EXA_TRY(d_dtmax.alloc(sizeof(unsigned long long)));
@@ -673,7 +665,7 @@ extern "C" int exa_musclhancock_solution_update(const exa_solver* s, double* luh
   EXA_TRY(hipMemcpy(d_lim.p, luh, sizeof(double) * patch, hipMemcpyHostToDevice));
   EXA_TRY(hipMemcpy(d_lim.d() + patch, luh_new, sizeof(double) * patch, hipMemcpyHostToDevice));
   EXA_TRY(hipMemset(d_cur.p, 0, 1));
-  EXA_TRY(hipMemset(d_flags.p, 0, sizeof(int) * 4));
+  EXA_TRY(hipMemset(d_flags.p, 0, sizeof(int) * exa::kLimFlags));
   EXA_TRY(hipMemcpy(d_dx.p, dx, sizeof(double) * 3, hipMemcpyHostToDevice));
   EXA_TRY(hipMemcpy(d_state.p, &dt, sizeof(double), hipMemcpyHostToDevice));  // StepState::dt is first
   exa::LimArgs a{};
