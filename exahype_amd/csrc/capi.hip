@@ -55,55 +55,41 @@ static int predictor_impl(const exa_solver* s, long ncells, double* lQhbnd, doub
   if (sd.linear || !exa::supported(sd) || sd.precision != exa::kFP64) return EXA_E_UNSUPPORTED;
   const Sizes z(sd);
   const bool exp = lQi || lFi || lQhi || lFhi;
-  DevBuf d_luh, d_qb, d_fb, d_du, d_dx, d_dt, d_it, d_qi, d_fi, d_qhi, d_fhi;
-  EXA_TRY(d_luh.alloc(sizeof(double) * ncells * z.B3 * z.D));
-  EXA_TRY(d_qb.alloc(sizeof(double) * ncells * 6 * z.B2 * z.D));
-  EXA_TRY(d_fb.alloc(sizeof(double) * ncells * 6 * z.B2 * z.V));
-  EXA_TRY(d_du.alloc(sizeof(double) * ncells * z.B3 * z.V));
-  EXA_TRY(d_dx.alloc(sizeof(double) * ncells * 3));
-  EXA_TRY(d_dt.alloc(sizeof(double)));
-  EXA_TRY(d_it.alloc(sizeof(int) * ncells));
-  if (exp) {
-    EXA_TRY(d_qi.alloc(sizeof(double) * ncells * z.B4 * z.D));
-    EXA_TRY(d_fi.alloc(sizeof(double) * ncells * 4 * z.B4 * z.V));
-    EXA_TRY(d_qhi.alloc(sizeof(double) * ncells * z.B3 * z.D));
-    EXA_TRY(d_fhi.alloc(sizeof(double) * ncells * 4 * z.B3 * z.V));
-    EXA_TRY(hipMemset(d_fi.p, 0, sizeof(double) * ncells * 4 * z.B4 * z.V));
-    EXA_TRY(hipMemset(d_fhi.p, 0, sizeof(double) * ncells * 4 * z.B3 * z.V));
-  }
-  EXA_TRY(hipMemcpy(d_luh.p, luh, sizeof(double) * ncells * z.B3 * z.D, hipMemcpyHostToDevice));
-  EXA_TRY(hipMemcpy(d_dx.p, dx, sizeof(double) * ncells * 3, hipMemcpyHostToDevice));
-  EXA_TRY(hipMemcpy(d_dt.p, &dt, sizeof(double), hipMemcpyHostToDevice));
+  const size_t w = sizeof(double) * ncells;
+  const int variant = exp ? exa::kPredictorValu144 : exa::kPredictorAuto;
+  const long ws_cells = std::min(ncells, exa::kPredictorWsCells);
+  const size_t wsb = exa::predictor_ws_bytes_per_cell(sd, variant) * ws_cells;
+  CallBuffers buf;
+  const int b_luh = buf.in(luh, w * z.B3 * z.D), b_dx = buf.in(dx, w * 3), b_dt = buf.in(&dt, sizeof(double));
+  const int b_qb = buf.out(lQhbnd, w * 6 * z.B2 * z.D), b_fb = buf.out(lFhbnd, w * 6 * z.B2 * z.V);
+  const int b_du = lduh ? buf.out(lduh, w * z.B3 * z.V) : -1, b_it = buf.out(iters, sizeof(int) * ncells);
+  const int b_qi = exp ? buf.out(lQi, w * z.B4 * z.D) : -1, b_qhi = exp ? buf.out(lQhi, w * z.B3 * z.D) : -1;
+  const int b_fi = exp ? buf.out(lFi, w * 4 * z.B4 * z.V, true) : -1;
+  const int b_fhi = exp ? buf.out(lFhi, w * 4 * z.B3 * z.V, true) : -1;
+  const int b_ws = wsb ? buf.scratch(wsb) : -1;
+  EXA_TRY(buf.up());
   exa::PredictorArgs a{};
-  a.luh = d_luh.d();
-  a.lduh = lduh ? d_du.d() : nullptr;
-  a.lQhbnd = d_qb.d();
-  a.lFhbnd = d_fb.d();
-  a.dx = d_dx.d();
+  a.luh = buf.d(b_luh);
+  a.lduh = lduh ? buf.d(b_du) : nullptr;
+  a.lQhbnd = buf.d(b_qb);
+  a.lFhbnd = buf.d(b_fb);
+  a.dx = buf.d(b_dx);
   a.dx_stride = 3;
-  a.dt = d_dt.d();
-  a.iters = static_cast<int*>(d_it.p);
+  a.dt = buf.d(b_dt);
+  a.iters = buf.as<int>(b_it);
   a.cell0 = 0;
-  a.lQi = d_qi.d();
-  a.lFi = d_fi.d();
-  a.lQhi = d_qhi.d();
-  a.lFhi = d_fhi.d();
-  DevBuf d_ws;
-  if (const size_t wsb = exa::predictor_ws_bytes_per_cell(sd, exp ? exa::kPredictorValu144 : exa::kPredictorAuto)) {
-    a.ws_cells = std::min(ncells, exa::kPredictorWsCells);
-    EXA_TRY(d_ws.alloc(wsb * a.ws_cells));
-    a.ws = d_ws.p;
+  if (exp) {
+    a.lQi = buf.d(b_qi);
+    a.lFi = buf.d(b_fi);
+    a.lQhi = buf.d(b_qhi);
+    a.lFhi = buf.d(b_fhi);
+  }
+  if (wsb) {
+    a.ws = buf.as<void>(b_ws);
+    a.ws_cells = ws_cells;
   }
   EXA_TRY(exa::launch_predictor(sd, exp, a, ncells, nullptr));
-  EXA_TRY(hipDeviceSynchronize());
-  EXA_TRY(hipMemcpy(lQhbnd, d_qb.p, sizeof(double) * ncells * 6 * z.B2 * z.D, hipMemcpyDeviceToHost));
-  EXA_TRY(hipMemcpy(lFhbnd, d_fb.p, sizeof(double) * ncells * 6 * z.B2 * z.V, hipMemcpyDeviceToHost));
-  if (lduh) EXA_TRY(hipMemcpy(lduh, d_du.p, sizeof(double) * ncells * z.B3 * z.V, hipMemcpyDeviceToHost));
-  if (iters) EXA_TRY(hipMemcpy(iters, d_it.p, sizeof(int) * ncells, hipMemcpyDeviceToHost));
-  if (lQi) EXA_TRY(hipMemcpy(lQi, d_qi.p, sizeof(double) * ncells * z.B4 * z.D, hipMemcpyDeviceToHost));
-  if (lFi) EXA_TRY(hipMemcpy(lFi, d_fi.p, sizeof(double) * ncells * 4 * z.B4 * z.V, hipMemcpyDeviceToHost));
-  if (lQhi) EXA_TRY(hipMemcpy(lQhi, d_qhi.p, sizeof(double) * ncells * z.B3 * z.D, hipMemcpyDeviceToHost));
-  if (lFhi) EXA_TRY(hipMemcpy(lFhi, d_fhi.p, sizeof(double) * ncells * 4 * z.B3 * z.V, hipMemcpyDeviceToHost));
+  EXA_TRY(buf.down());
   return EXA_OK;
 }
 
@@ -128,22 +114,17 @@ extern "C" int exa_volume_integral_nonlinear(const exa_solver* s, double* lduh, 
   if (!to_desc(s, &sd) || !lduh || !lFhi || !dx) return EXA_E_INVALID;
   if (sd.linear || !exa::supported_sizes(sd) || sd.precision != exa::kFP64) return EXA_E_UNSUPPORTED;
   const Sizes z(sd);
-  DevBuf d_du, d_fhi, d_dx, d_fi;
-  EXA_TRY(d_du.alloc(sizeof(double) * z.B3 * z.V));
-  EXA_TRY(d_fhi.alloc(sizeof(double) * 4 * z.B3 * z.V));
-  EXA_TRY(d_dx.alloc(sizeof(double) * 3));
-  if (sd.no_time_averaging) {  // the argument is lFi: average it over time first
-    EXA_TRY(d_fi.alloc(sizeof(double) * 4 * z.B3 * z.B * z.V));
-    EXA_TRY(hipMemcpy(d_fi.p, lFhi, sizeof(double) * 4 * z.B3 * z.B * z.V, hipMemcpyHostToDevice));
-    EXA_TRY(exa::launch_time_average_lfi(sd.order, z.V, d_fi.d(), d_fhi.d(), nullptr));
-  } else {
-    EXA_TRY(hipMemcpy(d_fhi.p, lFhi, sizeof(double) * 4 * z.B3 * z.V, hipMemcpyHostToDevice));
-  }
-  EXA_TRY(hipMemcpy(d_dx.p, dx, sizeof(double) * 3, hipMemcpyHostToDevice));
-  exa::VolumeArgs a{d_du.d(), d_fhi.d(), d_dx.d(), 0};
+  const size_t fhi = sizeof(double) * 4 * z.B3 * z.V;
+  CallBuffers buf;
+  const int b_du = buf.out(lduh, sizeof(double) * z.B3 * z.V), b_dx = buf.in(dx, sizeof(double) * 3);
+  // without time averaging the argument is lFi, which is averaged over time first
+  const int b_fi = sd.no_time_averaging ? buf.in(lFhi, fhi * z.B) : -1;
+  const int b_fhi = sd.no_time_averaging ? buf.scratch(fhi) : buf.in(lFhi, fhi);
+  EXA_TRY(buf.up());
+  if (sd.no_time_averaging) EXA_TRY(exa::launch_time_average_lfi(sd.order, z.V, buf.d(b_fi), buf.d(b_fhi), nullptr));
+  exa::VolumeArgs a{buf.d(b_du), buf.d(b_fhi), buf.d(b_dx), 0};
   EXA_TRY(exa::launch_volume_integral(sd, a, 1, nullptr));
-  EXA_TRY(hipDeviceSynchronize());
-  EXA_TRY(hipMemcpy(lduh, d_du.p, sizeof(double) * z.B3 * z.V, hipMemcpyDeviceToHost));
+  EXA_TRY(buf.down());
   return EXA_OK;
 }
 
@@ -166,37 +147,30 @@ static int update_impl(const exa_solver* s, int mode, double* luh, double* lduh,
   }
   const Sizes z(sd);
   const double one[3] = {1.0, 1.0, 1.0};
-  DevBuf d_luh, d_du, d_fb, d_dx, d_dt, d_cell;
-  EXA_TRY(d_luh.alloc(sizeof(double) * z.B3 * z.D));
-  EXA_TRY(d_du.alloc(sizeof(double) * z.B3 * z.V));
-  EXA_TRY(d_fb.alloc(sizeof(double) * 6 * z.B2 * z.V));
-  EXA_TRY(d_dx.alloc(sizeof(double) * 3));
-  EXA_TRY(d_dt.alloc(sizeof(double)));
-  EXA_TRY(d_cell.alloc(sizeof(double)));
-  EXA_TRY(hipMemset(d_luh.p, 0, sizeof(double) * z.B3 * z.D));
-  EXA_TRY(hipMemset(d_du.p, 0, sizeof(double) * z.B3 * z.V));
-  EXA_TRY(hipMemset(d_fb.p, 0, sizeof(double) * 6 * z.B2 * z.V));
-  if (luh) EXA_TRY(hipMemcpy(d_luh.p, luh, sizeof(double) * z.B3 * z.D, hipMemcpyHostToDevice));
-  if (lduh) EXA_TRY(hipMemcpy(d_du.p, lduh, sizeof(double) * z.B3 * z.V, hipMemcpyHostToDevice));
-  if (lFhbnd) EXA_TRY(hipMemcpy(d_fb.p, lFhbnd, sizeof(double) * 6 * z.B2 * z.V, hipMemcpyHostToDevice));
-  EXA_TRY(hipMemcpy(d_dx.p, dx ? dx : one, sizeof(double) * 3, hipMemcpyHostToDevice));
-  EXA_TRY(hipMemcpy(d_dt.p, &dt, sizeof(double), hipMemcpyHostToDevice));
+  CallBuffers buf;
+  const size_t n_luh = sizeof(double) * z.B3 * z.D, n_du = sizeof(double) * z.B3 * z.V;
+  // absent arguments are zeros
+  const int b_luh = mode & exa::kUpdUpdate ? buf.inout(luh, luh, n_luh) : (luh ? buf.in(luh, n_luh) : buf.zeroed(n_luh));
+  const int b_du =
+      mode & exa::kUpdWriteLduh ? buf.inout(lduh, lduh, n_du) : (lduh ? buf.in(lduh, n_du) : buf.zeroed(n_du));
+  const size_t n_fb = sizeof(double) * 6 * z.B2 * z.V;
+  const int b_fb = lFhbnd ? buf.in(lFhbnd, n_fb) : buf.zeroed(n_fb);
+  const int b_dx = buf.in(dx ? dx : one, sizeof(double) * 3), b_dt = buf.in(&dt, sizeof(double));
+  const int b_cell = dt_out ? buf.out(dt_out, sizeof(double)) : -1;
+  EXA_TRY(buf.up());
   exa::UpdateArgs a{};
-  a.luh = d_luh.d();
-  a.lduh = d_du.d();
-  a.lFhbnd = d_fb.d();
-  a.dx = d_dx.d();
+  a.luh = buf.d(b_luh);
+  a.lduh = buf.d(b_du);
+  a.lFhbnd = buf.d(b_fb);
+  a.dx = buf.d(b_dx);
   a.dx_stride = 0;
-  a.dt = d_dt.d();
+  a.dt = buf.d(b_dt);
   a.cfl_pnpm = sd.cfl * kPNPM[sd.order];
   a.dt_slots = nullptr;
-  a.dt_cell = dt_out ? d_cell.d() : nullptr;
+  a.dt_cell = dt_out ? buf.d(b_cell) : nullptr;
   a.cell0 = 0;
   EXA_TRY(exa::launch_update(sd, mode, a, 1, nullptr));
-  EXA_TRY(hipDeviceSynchronize());
-  if (mode & exa::kUpdUpdate) EXA_TRY(hipMemcpy(luh, d_luh.p, sizeof(double) * z.B3 * z.D, hipMemcpyDeviceToHost));
-  if (mode & exa::kUpdWriteLduh) EXA_TRY(hipMemcpy(lduh, d_du.p, sizeof(double) * z.B3 * z.V, hipMemcpyDeviceToHost));
-  if (dt_out) EXA_TRY(hipMemcpy(dt_out, d_cell.p, sizeof(double), hipMemcpyDeviceToHost));
+  EXA_TRY(buf.down());
   return EXA_OK;
 }
 
@@ -224,25 +198,28 @@ extern "C" int exa_riemann_solver_nonlinear(const exa_solver* s, double* FL, dou
   if (!to_desc(s, &sd) || !FL || !FR || !QL || !QR || direction < 0 || direction > 2) return EXA_E_INVALID;
   if (sd.linear || !exa::supported(sd) || sd.precision != exa::kFP64) return EXA_E_UNSUPPORTED;
   const Sizes z(sd);
-  // Two cells: cell 0 owns face 2d+1 (left state), cell 1 owns face 2d (right state).
-  DevBuf d_qb, d_fb, d_face;
+    // One cell's face blocks, with the left state at 2d+1 and the right one at 2d
+  // (as if the cell were its own neighbour).
   const long qf = z.B2 * z.D, ff = z.B2 * z.V;
-  EXA_TRY(d_qb.alloc(sizeof(double) * 2 * 6 * qf));
-  EXA_TRY(d_fb.alloc(sizeof(double) * 2 * 6 * ff));
-  EXA_TRY(d_face.alloc(sizeof(FaceDesc)));
-  const long iqL = (0 * 6 + 2 * direction + 1) * qf, iqR = (1 * 6 + 2 * direction) * qf;
-  const long ifL = (0 * 6 + 2 * direction + 1) * ff, ifR = (1 * 6 + 2 * direction) * ff;
-  EXA_TRY(hipMemcpy(d_qb.d() + iqL, QL, sizeof(double) * qf, hipMemcpyHostToDevice));
-  EXA_TRY(hipMemcpy(d_qb.d() + iqR, QR, sizeof(double) * qf, hipMemcpyHostToDevice));
-  EXA_TRY(hipMemcpy(d_fb.d() + ifL, FL, sizeof(double) * ff, hipMemcpyHostToDevice));
-  EXA_TRY(hipMemcpy(d_fb.d() + ifR, FR, sizeof(double) * ff, hipMemcpyHostToDevice));
-  const FaceDesc f{0, 1, direction, 0};
-  EXA_TRY(hipMemcpy(d_face.p, &f, sizeof(FaceDesc), hipMemcpyHostToDevice));
-  exa::RiemannArgs a{static_cast<const FaceDesc*>(d_face.p), 1, d_qb.d(), d_fb.d()};
+  constexpr long kMost = 64 * 16;  // B^2 D of every compiled solver is below
+  if (qf > kMost) return EXA_E_UNSUPPORTED;
+  double q[6 * kMost] = {}, F[6 * kMost] = {};
+  double *const q_right = q + 2 * direction * qf, *const q_left = q_right + qf;
+  double *const F_right = F + 2 * direction * ff, *const F_left = F_right + ff;
+  std::copy_n(QL, qf, q_left);
+  std::copy_n(QR, qf, q_right);
+  std::copy_n(FL, ff, F_left);
+  std::copy_n(FR, ff, F_right);
+  const FaceDesc f{0, 0, direction, 0};
+  CallBuffers buf;
+  const int b_q = buf.in(q, sizeof(double) * 6 * qf), b_f = buf.inout(F, F, sizeof(double) * 6 * ff);
+  const int b_face = buf.in(&f, sizeof(f));
+  EXA_TRY(buf.up());
+  exa::RiemannArgs a{buf.as<const FaceDesc>(b_face), 1, buf.d(b_q), buf.d(b_f)};
   EXA_TRY(exa::launch_riemann(sd, a, nullptr));
-  EXA_TRY(hipDeviceSynchronize());
-  EXA_TRY(hipMemcpy(FL, d_fb.d() + ifL, sizeof(double) * ff, hipMemcpyDeviceToHost));
-  EXA_TRY(hipMemcpy(FR, d_fb.d() + ifR, sizeof(double) * ff, hipMemcpyDeviceToHost));
+  EXA_TRY(buf.down());
+  std::copy_n(F_left, ff, FL);
+  std::copy_n(F_right, ff, FR);
   return EXA_OK;
 }
 
@@ -384,8 +361,7 @@ extern "C" int exa_riemann_solver_linear(const exa_solver* s, double* FL, double
   sd.linear = 1;
   if (!exa::linear_supported(sd)) return EXA_E_UNSUPPORTED;
   const Sizes z(sd);
-  // Two cells: cell 0 owns face 2d+1 (left state), cell 1 owns face 2d (right state).
-  DevBuf d_qb, d_fb, d_face;
+    DevBuf d_qb, d_fb, d_face;
   const long qf = z.B2 * z.D, ff = z.B2 * z.V;
   EXA_TRY(d_qb.alloc(sizeof(double) * 2 * 6 * qf));
   EXA_TRY(d_fb.alloc(sizeof(double) * 2 * 6 * ff));
