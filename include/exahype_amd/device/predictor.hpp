@@ -92,7 +92,13 @@ struct PredictorLayout {
   static constexpr long kOther =
       (long)(SF + (USE_NCP ? (IN_PLACE ? 0 : V * B3) + B2 : 0) + 3 + 2 * (NT / kWave)) * sizeof(T);
   static constexpr long kFree = kLdsBudget - kOther;
-  static constexpr int NQL = kFree <= 0 ? 0 : (kFree / kSliceBytes >= B ? B : (int)(kFree / kSliceBytes));
+  // Up to B = 4 a flux-only PDE's iterate fits the registers beside the next one
+  // (40 of 222 in double at B = 4): its reads and writes were a fifth of the LDS
+  // traffic that binds these sizes.  64,000 cells, double and float: N=3 0.96 ->
+  // 0.84 ms and 0.385 -> 0.342, N=2 0.543 -> 0.477 and 0.180 -> 0.147; N=4 loses
+  // a wavefront per SIMD (1.97 -> 2.62 ms) and keeps it in LDS.
+  static constexpr bool IN_REGISTERS = B <= 4 && V <= 5 && USE_FLUX && !USE_NCP;
+  static constexpr int NQL = kFree <= 0 || IN_REGISTERS ? 0 : (kFree / kSliceBytes >= B ? B : (int)(kFree / kSliceBytes));
   static constexpr int NQR = B - NQL;
   // Rolled slices: the large sizes and the 9-variable PDE, whose unrolled
   // slices exhaust the registers, and the float form at N=4 and N=5, where the
@@ -100,18 +106,17 @@ struct PredictorLayout {
   // wavefront per SIMD) at the cost of uniform table loads per slice
   // (measured: N=4 -2%, N=5 -4% predictor time; at N=6 the rolled form was
   // 19% slower, so N=6 stays unrolled), and the double form of the
-  // 5-variable PDE at N=3, where the rolled loop leaves room for the
-  // accumulated time averages (the predictor kernel's ACC_FH), and at N=5,
-  // whose unrolled slices beside the closed first iteration exceed the 256
+  // 5-variable PDE at N=5, whose unrolled slices beside the closed first iteration exceed the 256
   // registers of the two wavefronts per SIMD its LDS allows.
   static constexpr bool ROLLED = (B >= 7 && (IS_FP64 || B >= 8)) || V >= 9 || (!IS_FP64 && (B == 5 || B == 6)) ||
-                                 (IS_FP64 && (B == 4 || B == 6) && V == 5);
+                                 (IS_FP64 && B == 6 && V == 5);
   // 8+ waves per workgroup leave 256 registers per lane, no room for slices;
   // a rolled loop cannot index registers.
   static constexpr bool WSQ = NQR > 0 && (NT >= 8 * kWave || ROLLED);
   // unroll factor of the loop over time slices
   static constexpr int UNROLL_T = ROLLED ? 1 : B;
   static constexpr bool SPLIT = ROLLED && WSQ && NQL > 0;
+  static constexpr bool LINES = B == 4 && USE_FLUX;
   static constexpr size_t ws_bytes = WSQ ? (size_t)NQR * V * B3 * sizeof(T) : 0;
 };
 
@@ -182,6 +187,15 @@ __global__ __launch_bounds__(node_threads(B), (predictor_min_waves<B, PDE, TERMS
   const bool active = tid < B3;
   const int node = active ? tid : 0;
   const int z = node / B2, y = (node / B) % B, x = node % B;
+  // LINES: a direction's flux rows are kept by coordinate along the direction
+  // and then by line, each coordinate's lines turned by four places, instead of
+  // by node: node owners and line owners both touch every bank once.  By node
+  // the lines along x and y meet in a quarter of the banks at B = 4 (in double
+  // 1.04 -> 0.96 ms for 64,000 cells, 26 -> 24 us for 729).
+  constexpr bool LINES = L::LINES;
+  auto line_place = [](int n, int line) __device__ { return n * B2 + ((line + 4 * n) & (B2 - 1)); };
+  const int at[3] = {LINES ? line_place(x, z * B + y) : node, LINES ? line_place(y, z * B + x) : node,
+                     LINES ? line_place(z, y * B + x) : node};
   if (a.run_if && *a.run_if == 0) return;  // whole launch
   if (a.status && a.status[cell] >= a.status_limit) {  // whole workgroup
     if (a.iters && tid == 0) a.iters[cell] = 0;
@@ -248,12 +262,10 @@ __global__ __launch_bounds__(node_threads(B), (predictor_min_waves<B, PDE, TERMS
   // 8, where they fit the wavefronts per SIMD that LDS allows (B = 6 and 8
   // with the register cap of predictor_min_waves: 124 and 166 registers; the
   // epilogue's B flux evaluations go, 4% of the predictor at 81^3 N=5; B = 3
-  // and 4 would drop a wavefront per SIMD, B = 7 spills under the cap), and
-  // the double form of the 5-variable PDE at B = 4 with its slice loop rolled
-  // (170 registers, the two wavefronts per SIMD its LDS allows; 3.44 -> 3.36
-  // ms at 81^3 in the limiter workload, where one iteration is the rule)
-  constexpr bool ACC_FH = (FLOAT_FLUX_ONLY && (B == 5 || B == 6 || B == 8)) ||
-                          (IS_FP64 && USE_FLUX && !USE_SRC_NCP && B == 4 && V == 5);
+  // and 4 would drop a wavefront per SIMD, B = 7 spills under the cap; in
+  // double at B = 4, beside the iterate in registers, one wavefront per SIMD
+  // would be left: 0.89 -> 1.18 ms for 64,000 cells)
+  constexpr bool ACC_FH = FLOAT_FLUX_ONLY && (B == 5 || B == 6 || B == 8);
   T fh[3][V];
   // Float form of a PDE without fluxes (source and/or NCP only: the elastic
   // PDE): the time-averaged source term likewise accumulates during the
@@ -289,16 +301,19 @@ __global__ __launch_bounds__(node_threads(B), (predictor_min_waves<B, PDE, TERMS
         // line starts: x-lines (z,y) stride 1, y-lines (z,x) stride B,
         // z-lines (y,x) stride B^2
         const int off0 = m * B3 + line * B, off1 = m * B3 + la * B2 + lb, off2 = m * B3 + line;
+        int off[B];
+#pragma unroll
+        for (int n = 0; n < B; ++n) off[n] = LINES ? m * B3 + line_place(n, line) : 0;
 #pragma unroll
         for (int d = 0; d < 3; ++d) {
           const int stride = d == 0 ? 1 : (d == 1 ? B : B2);
-          const int o = d * V * B3 + (d == 0 ? off0 : (d == 1 ? off1 : off2));
+          const int o = d * V * B3 + (LINES ? 0 : (d == 0 ? off0 : (d == 1 ? off1 : off2)));
           T f[B], out[B];
 #pragma unroll
-          for (int n = 0; n < B; ++n) f[n] = sF[o + n * stride];
+          for (int n = 0; n < B; ++n) f[n] = sF[LINES ? o + off[n] : o + n * stride];
           contract_halves<B, VOLUME>(f, out);
 #pragma unroll
-          for (int l = 0; l < B; ++l) sF[o + l * stride] = out[l];
+          for (int l = 0; l < B; ++l) sF[LINES ? o + off[l] : o + l * stride] = out[l];
         }
       }
     }
@@ -364,7 +379,7 @@ __global__ __launch_bounds__(node_threads(B), (predictor_min_waves<B, PDE, TERMS
 #pragma unroll
           for (int d = 0; d < 3; ++d)
 #pragma unroll
-            for (int m = 0; m < V; ++m) sF[(d * V + m) * B3 + node] = F[d][m];
+            for (int m = 0; m < V; ++m) sF[(d * V + m) * B3 + at[d]] = F[d][m];
           if (EXPORT) {
             double* lFi = a.lFi + cell * (size_t)(4 * B3 * B * V) + (((size_t)t * B3 + node) * 4) * V;
 #pragma unroll
@@ -392,9 +407,9 @@ __global__ __launch_bounds__(node_threads(B), (predictor_min_waves<B, PDE, TERMS
       for (int m = 0; m < V; ++m) {
         ir[m] = IN_PLACE ? T(0) : fl_t * q0i[m];
         if (USE_FLUX) {
-          ir[m] -= wg[0] * sF[(0 * V + m) * B3 + node];
-          ir[m] -= wg[1] * sF[(1 * V + m) * B3 + node];
-          ir[m] -= wg[2] * sF[(2 * V + m) * B3 + node];
+          ir[m] -= wg[0] * sF[(0 * V + m) * B3 + at[0]];
+          ir[m] -= wg[1] * sF[(1 * V + m) * B3 + at[1]];
+          ir[m] -= wg[2] * sF[(2 * V + m) * B3 + at[2]];
         }
       }
       if (USE_SRC_NCP) {
@@ -443,7 +458,7 @@ __global__ __launch_bounds__(node_threads(B), (predictor_min_waves<B, PDE, TERMS
         for (int d = 0; d < 3; ++d)
 #pragma unroll
           for (int m = 0; m < V; ++m) {
-            sF[(d * V + m) * B3 + node] = F[d][m];
+            sF[(d * V + m) * B3 + at[d]] = F[d][m];
             if constexpr (ACC_FH) fh[d][m] = F[d][m] * sumw;
           }
       }
@@ -455,8 +470,8 @@ __global__ __launch_bounds__(node_threads(B), (predictor_min_waves<B, PDE, TERMS
       if constexpr (USE_FLUX) contract_lines.template operator()<false>();
 #pragma unroll
       for (int m = 0; m < V; ++m)
-        R[m] = USE_FLUX ? gd[0] * sF[(0 * V + m) * B3 + node] + gd[1] * sF[(1 * V + m) * B3 + node] +
-                              gd[2] * sF[(2 * V + m) * B3 + node]
+        R[m] = USE_FLUX ? gd[0] * sF[(0 * V + m) * B3 + at[0]] + gd[1] * sF[(1 * V + m) * B3 + at[1]] +
+                              gd[2] * sF[(2 * V + m) * B3 + at[2]]
                         : T(0);
       if constexpr (USE_SRC_NCP) {
         T S[V];
@@ -584,7 +599,7 @@ __global__ __launch_bounds__(node_threads(B), (predictor_min_waves<B, PDE, TERMS
           T accL = T(0), accR = T(0);
 #pragma unroll
           for (int l = 0; l < B; ++l) {
-            const T v = sF[o + l * stride];
+            const T v = sF[LINES && PER_DIR ? (d * V + k) * B3 + line_place(l, line) : o + l * stride];
             accL += v * tc<T>(exa_fl_coeff[N][l]);
             accR += v * tc<T>(exa_fr_coeff[N][l]);
           }
@@ -664,7 +679,7 @@ __global__ __launch_bounds__(node_threads(B), (predictor_min_waves<B, PDE, TERMS
 #pragma unroll
     for (int d = 0; d < 3; ++d)
 #pragma unroll
-      for (int m = 0; m < V; ++m) sF[(d * V + m) * B3 + node] = fh[d][m];
+      for (int m = 0; m < V; ++m) sF[(d * V + m) * B3 + at[d]] = fh[d][m];
     __syncthreads();
   }
   // lFhbnd from lFhi_{x,y,z} (:434-527)
@@ -688,8 +703,8 @@ __global__ __launch_bounds__(node_threads(B), (predictor_min_waves<B, PDE, TERMS
       const T us[3] = {wz * wy * invDx[0], wz * wx * invDx[1], wy * wx * invDx[2]};
 #pragma unroll
       for (int m = 0; m < V; ++m)
-        acc[m] = us[0] * sF[(0 * V + m) * B3 + node] + us[1] * sF[(1 * V + m) * B3 + node] +
-                 us[2] * sF[(2 * V + m) * B3 + node];
+        acc[m] = us[0] * sF[(0 * V + m) * B3 + at[0]] + us[1] * sF[(1 * V + m) * B3 + at[1]] +
+                 us[2] * sF[(2 * V + m) * B3 + at[2]];
     }
     if (USE_SRC_NCP) {
 #pragma unroll
