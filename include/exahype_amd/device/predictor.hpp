@@ -116,7 +116,7 @@ struct PredictorLayout {
   // unroll factor of the loop over time slices
   static constexpr int UNROLL_T = ROLLED ? 1 : B;
   static constexpr bool SPLIT = ROLLED && WSQ && NQL > 0;
-  static constexpr bool LINES = B == 4 && USE_FLUX;
+  static constexpr bool LINES = USE_FLUX && (B == 4 || (B == 8 && LDSK == 144 && !USE_NCP));
   static constexpr size_t ws_bytes = WSQ ? (size_t)NQR * V * B3 * sizeof(T) : 0;
 };
 
@@ -188,14 +188,16 @@ __global__ __launch_bounds__(node_threads(B), (predictor_min_waves<B, PDE, TERMS
   const int node = active ? tid : 0;
   const int z = node / B2, y = (node / B) % B, x = node % B;
   // LINES: a direction's flux rows are kept by coordinate along the direction
-  // and then by line, each coordinate's lines turned by four places, instead of
-  // by node: node owners and line owners both touch every bank once.  By node
-  // the lines along x and y meet in a quarter of the banks at B = 4 (in double
-  // 1.04 -> 0.96 ms for 64,000 cells, 26 -> 24 us for 729).
+  // and then by line, each coordinate's lines turned by four places (x) or B,
+  // instead of by node: node owners and line owners both touch every bank once.
+  // By node the lines along x and y meet in a quarter of the banks: B = 4 in
+  // double 1.04 -> 0.96 ms for 64,000 cells, B = 8 in float 1.65 -> 1.53 ms for
+  // 20,000, in double 4.90 -> 4.79 ms for 15,000.  (Not at B = 8 with the 64 KB
+  // budget or the non-conservative product, which have no registers for it.)
   constexpr bool LINES = L::LINES;
-  auto line_place = [](int n, int line) __device__ { return n * B2 + ((line + 4 * n) & (B2 - 1)); };
-  const int at[3] = {LINES ? line_place(x, z * B + y) : node, LINES ? line_place(y, z * B + x) : node,
-                     LINES ? line_place(z, y * B + x) : node};
+  auto line_place = [](int d, int n, int line) __device__ { return n * B2 + ((line + (d == 0 ? 4 : B) * n) & (B2 - 1)); };
+  const int at[3] = {LINES ? line_place(0, x, z * B + y) : node, LINES ? line_place(1, y, z * B + x) : node,
+                     LINES ? line_place(2, z, y * B + x) : node};
   if (a.run_if && *a.run_if == 0) return;  // whole launch
   if (a.status && a.status[cell] >= a.status_limit) {  // whole workgroup
     if (a.iters && tid == 0) a.iters[cell] = 0;
@@ -301,19 +303,16 @@ __global__ __launch_bounds__(node_threads(B), (predictor_min_waves<B, PDE, TERMS
         // line starts: x-lines (z,y) stride 1, y-lines (z,x) stride B,
         // z-lines (y,x) stride B^2
         const int off0 = m * B3 + line * B, off1 = m * B3 + la * B2 + lb, off2 = m * B3 + line;
-        int off[B];
-#pragma unroll
-        for (int n = 0; n < B; ++n) off[n] = LINES ? m * B3 + line_place(n, line) : 0;
 #pragma unroll
         for (int d = 0; d < 3; ++d) {
           const int stride = d == 0 ? 1 : (d == 1 ? B : B2);
           const int o = d * V * B3 + (LINES ? 0 : (d == 0 ? off0 : (d == 1 ? off1 : off2)));
           T f[B], out[B];
 #pragma unroll
-          for (int n = 0; n < B; ++n) f[n] = sF[LINES ? o + off[n] : o + n * stride];
+          for (int n = 0; n < B; ++n) f[n] = sF[LINES ? o + m * B3 + line_place(d, n, line) : o + n * stride];
           contract_halves<B, VOLUME>(f, out);
 #pragma unroll
-          for (int l = 0; l < B; ++l) sF[LINES ? o + off[l] : o + l * stride] = out[l];
+          for (int l = 0; l < B; ++l) sF[LINES ? o + m * B3 + line_place(d, l, line) : o + l * stride] = out[l];
         }
       }
     }
@@ -599,7 +598,7 @@ __global__ __launch_bounds__(node_threads(B), (predictor_min_waves<B, PDE, TERMS
           T accL = T(0), accR = T(0);
 #pragma unroll
           for (int l = 0; l < B; ++l) {
-            const T v = sF[LINES && PER_DIR ? (d * V + k) * B3 + line_place(l, line) : o + l * stride];
+            const T v = sF[LINES && PER_DIR ? (d * V + k) * B3 + line_place(d, l, line) : o + l * stride];
             accL += v * tc<T>(exa_fl_coeff[N][l]);
             accR += v * tc<T>(exa_fr_coeff[N][l]);
           }
