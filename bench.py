@@ -492,7 +492,7 @@ def bench_amr(capi, args):
         "restrict_after_prolong_max_err": err,
         "roofline": dict(bound="hbm", achieved=round(achieved, 1), peak=HBM_PEAK_GBS, unit="GB/s",
                          frac=round(achieved / HBM_PEAK_GBS, 4), traffic=amr_measured_traffic("prolongation"),
-                         kernel="amr_kernel<6,3,false> (volume prolongation, one level)",
+                         kernel="amr_prolong_kernel<6,3> (volume prolongation, one level)",
                          avg_launch_ms=round(p_ms, 4), algorithmic_bytes_per_launch=alg_p,
                          restriction={"avg_launch_ms": round(r_ms, 4), "algorithmic_bytes_per_launch": alg_r,
                                       "achieved_GBs": round(alg_r / (r_ms * 1e-3) / 1e9, 1),
