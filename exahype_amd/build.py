@@ -106,11 +106,11 @@ USER_EXAMPLE = os.path.join(HERE, "libexa_user_example.so")
 
 
 def build_user_example(verbose=False):
-    """A user's PDE compiled into the device kernels through
-    include/exahype_amd/user_solver.hpp, as a user would build it: its own
-    shared object, independent of the library's."""
-    src = os.path.join(HERE, "examples", "user_euler.hip")
-    cmd = [hipcc()] + HIPCC_FLAGS + ["-Rpass-analysis=kernel-resource-usage", "-o", USER_EXAMPLE + ".tmp", src]
+    """Users' PDEs compiled into the device kernels through
+    include/exahype_amd/user_solver.hpp, as a user would build them: a shared
+    object of their own, independent of the library's."""
+    srcs = [os.path.join(HERE, "examples", s) for s in ("user_euler.hip", "user_linear.hip")]
+    cmd = [hipcc()] + HIPCC_FLAGS + ["-Rpass-analysis=kernel-resource-usage", "-o", USER_EXAMPLE + ".tmp"] + srcs
     if verbose:
         print(" ".join(cmd), flush=True)
     res = subprocess.run(cmd, capture_output=True, text=True)

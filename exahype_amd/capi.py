@@ -519,10 +519,12 @@ _user_example = None
 
 
 def user_example():
-    """The example user solver (examples/user_euler.hip): an Euler PDE with a
-    reflecting-wall boundaryValues and an entropy-wave adjustPointSolution,
-    compiled through include/exahype_amd/user_solver.hpp into its own shared
-    object.  Tables: exa_user_euler_order3, exa_user_euler_order5."""
+    """The example user solvers, compiled through
+    include/exahype_amd/user_solver.hpp into their own shared object.  Tables:
+    exa_user_euler_order3, exa_user_euler_order5 (examples/user_euler.hip: an
+    Euler PDE with a reflecting-wall boundaryValues and an entropy-wave
+    adjustPointSolution) and those of examples/user_linear.hip (PDEs with a
+    non-conservative product)."""
     global _user_example
     if _user_example is None:
         if not os.path.exists(USER_EXAMPLE_PATH):

@@ -85,7 +85,9 @@ struct PredictorLayout {
   static constexpr int NT = node_threads(B);
   static constexpr bool IS_FP64 = sizeof(T) == sizeof(double);
   static constexpr long kLdsBudget = (long)LDSK * 1024;
-  static constexpr bool IN_PLACE = USE_NCP && !USE_FLUX && (long)(B * V * B3 + B2 + 64) * (long)sizeof(T) <= kLdsBudget;
+  // (its B V rows also take the epilogue's D: not with parameters beyond (B - 1) V)
+  static constexpr bool IN_PLACE = USE_NCP && !USE_FLUX && B * V >= D &&
+                                   (long)(B * V * B3 + B2 + 64) * (long)sizeof(T) <= kLdsBudget;
   // LDS: one slice of fluxes [dir][var][node] (reused for lQhi / lFhi staging)
   static constexpr int SF = IN_PLACE ? 0 : (3 * V > D ? 3 * V : D) * B3;
   static constexpr long kSliceBytes = (long)V * B3 * sizeof(T);
@@ -107,9 +109,10 @@ struct PredictorLayout {
   // (measured: N=4 -2%, N=5 -4% predictor time; at N=6 the rolled form was
   // 19% slower, so N=6 stays unrolled), and the double form of the
   // 5-variable PDE at N=5, whose unrolled slices beside the closed first iteration exceed the 256
-  // registers of the two wavefronts per SIMD its LDS allows.
+  // registers of the two wavefronts per SIMD its LDS allows (with so many parameters that LDS does
+  // not hold all slices, they stay unrolled: a user's solver has no workspace).
   static constexpr bool ROLLED = (B >= 7 && (IS_FP64 || B >= 8)) || V >= 9 || (!IS_FP64 && (B == 5 || B == 6)) ||
-                                 (IS_FP64 && B == 6 && V == 5);
+                                 (IS_FP64 && B == 6 && V == 5 && (NQR == 0 || LDSK < 144));
   // 8+ waves per workgroup leave 256 registers per lane, no room for slices;
   // a rolled loop cannot index registers.
   static constexpr bool WSQ = NQR > 0 && (NT >= 8 * kWave || ROLLED);

@@ -18,7 +18,7 @@ import ctypes
 import numpy as np
 import pytest
 
-from refutil import rel_per_dof
+from refutil import elastic_cells, rel_per_dof
 
 pytestmark = pytest.mark.gpu
 
@@ -147,6 +147,35 @@ def test_fp32_bulk_user_grid(exa):
     l2 = np.linalg.norm(out[1] - out[0]) / np.linalg.norm(out[0])
     print(f"  L2 {l2:.2e}", flush=True)
     assert l2 < 1e-6
+
+
+@pytest.mark.parametrize("name,order,n,steps,npar", [("order1_many", 1, 5, 6, 10), ("order2", 2, 4, 6, 3),
+                                                     ("order4", 4, 3, 4, 3)])
+def test_flux_free_user_pde_vs_oracle(exa, oracle, name, order, n, steps, npar):
+    """Elasticity as a user's PDE (a non-conservative product and no flux):
+    gradients from the iterate in place, or from a staged slice where the
+    parameters outnumber the iterate's rows.  Bars of the library's elastic grid."""
+    print(f"case: flux-free user PDE {name} {n}^3", flush=True)
+    nodes = np.array([oracle.table(oracle.T_NODES, order, i) for i in range(order + 1)])
+    luh = elastic_cells(order, n, seed=5, nodes=nodes, width=0.15).reshape(-1, 12)
+    extra = np.random.default_rng(order).uniform(-1, 1, (len(luh), npar - 3))
+    o = oracle.Grid(oracle.elastic_solver(order), n)
+    o.set_solution(luh.ravel())
+    odts, _ = o.step(steps)
+    want = np.concatenate([o.solution().reshape(-1, 12), extra], 1)
+    for precision, tol in ((exa.PRECISION_FP64, 1e-12), (exa.PRECISION_FP32_BULK, None)):
+        g = exa.Grid.from_user_solver(getattr(exa.user_example(), f"exa_user_elastic_{name}"), n, precision=precision)
+        g.upload(np.concatenate([luh, extra], 1).ravel())
+        g.step(steps)
+        got = g.solution().reshape(-1, 9 + npar)
+        assert np.array_equal(got[:, 9:], want[:, 9:])
+        if tol:
+            assert np.abs(g.dt_history(steps) - odts).max() <= 1e-13 * odts.max()
+            assert np.array_equal(g.picard_iterations(), o.picard_iterations())
+            assert (np.abs(got - want).max(axis=0) <= tol * np.abs(want).max(axis=0)).all()
+        else:
+            assert np.linalg.norm(got[:, :9] - want[:, :9]) <= 1e-5 * np.linalg.norm(want[:, :9])
+        g.close()
 
 
 def test_user_route_refusals(exa):
