@@ -47,9 +47,69 @@ struct UserElastic {
   }
 };
 
+// Linear acoustics with a tracer carried by a constant wind (variables
+// pressure, u, v, w, tracer).  SPLIT: half of every term as a flux and half as a
+// non-conservative product, which for constant coefficients are the same
+// operator, so that both forms compute the same solution.
+template <bool SPLIT>
+struct UserWaves {
+  static constexpr int V = 5;
+  static constexpr int P = 0;
+  static constexpr double CFL = 0.05;  // the Picard iteration ends by its residual, not its limit
+
+  template <typename T>
+  __device__ static T wind(int d) {
+    return d == 0 ? T(0.5) : (d == 1 ? T(-0.25) : T(0.75));
+  }
+
+  // A_d q: density 2, bulk modulus 3
+  template <typename T>
+  __device__ static void apply(int d, const T* q, T* out) {
+    out[0] = T(3) * q[1 + d] + wind<T>(d) * q[0];
+    for (int k = 0; k < 3; ++k) out[1 + k] = wind<T>(d) * q[1 + k] + (k == d ? T(0.5) * q[0] : T(0));
+    out[4] = wind<T>(d) * q[4];
+  }
+
+  template <typename T>
+  __device__ static void flux(const T* Q, T (*F)[V]) {
+    for (int d = 0; d < 3; ++d) {
+      apply(d, Q, F[d]);
+      if (SPLIT)
+        for (int m = 0; m < V; ++m) F[d][m] *= T(0.5);
+    }
+  }
+
+  template <typename T>
+  __device__ static void eigenvalues(const T*, int d, T* lambda) {
+    const T c = sqrt(T(1.5));
+    for (int m = 0; m < V; ++m) lambda[m] = wind<T>(d);
+    lambda[0] -= c;
+    lambda[1] += c;
+  }
+
+  template <typename T>
+  __device__ static void algebraic_source(const T*, T* S) {
+    for (int m = 0; m < V; ++m) S[m] = T(0);
+  }
+
+  template <typename T>
+  __device__ static void ncp(const T*, const T (*g)[V], T* BgradQ) {
+    T a[3][V];
+    for (int d = 0; d < 3; ++d) apply(d, g[d], a[d]);
+    for (int m = 0; m < V; ++m) BgradQ[m] = T(0.5) * (a[0][m] + a[1][m] + a[2][m]);
+  }
+};
+
 }  // namespace
 
 // at order 1 the parameters outnumber the rows of the predictor's iterate
 EXA_USER_SOLVER(exa_user_elastic_order1_many, UserElastic<7>, 1, exa::kNCP)
 EXA_USER_SOLVER(exa_user_elastic_order2, UserElastic<0>, 2, exa::kNCP)
 EXA_USER_SOLVER(exa_user_elastic_order4, UserElastic<0>, 4, exa::kNCP)
+EXA_USER_SOLVER(exa_user_waves_order3, UserWaves<false>, 3, exa::kFlux)
+EXA_USER_SOLVER(exa_user_waves_order4, UserWaves<false>, 4, exa::kFlux)
+EXA_USER_SOLVER(exa_user_waves_order5, UserWaves<false>, 5, exa::kFlux)
+EXA_USER_SOLVER(exa_user_waves_split_order3, UserWaves<true>, 3, exa::kFlux | exa::kNCP)
+EXA_USER_SOLVER(exa_user_waves_split_order4, UserWaves<true>, 4, exa::kFlux | exa::kNCP | exa::kSource)
+EXA_USER_SOLVER(exa_user_waves_split_order5, UserWaves<true>, 5, exa::kFlux | exa::kNCP)
+EXA_USER_SOLVER(exa_user_waves_source_order4, UserWaves<false>, 4, exa::kFlux | exa::kSource)

@@ -79,7 +79,8 @@ __device__ inline void source_ncp(const T* Q, const T* sQ, const T* sDu, const T
 // double, 41^3 cells, 8 steps: predictor 4.08 -> 2.26 ms per step together
 // with the closed first iteration, the whole run 51.1 -> 46.7 ms by this form
 // and the boundary fluxes left out.
-template <int B, int V, int D, bool USE_NCP, typename T, int LDSK = 144, bool USE_FLUX = true>
+template <int B, int V, int D, bool USE_NCP, typename T, int LDSK = 144, bool USE_FLUX = true,
+          bool USE_SOURCE = false>
 struct PredictorLayout {
   static constexpr int B2 = B * B, B3 = B2 * B;
   static constexpr int NT = node_threads(B);
@@ -107,12 +108,22 @@ struct PredictorLayout {
   // rolled loop needs fewer registers (N=5: 110 instead of 166, one more
   // wavefront per SIMD) at the cost of uniform table loads per slice
   // (measured: N=4 -2%, N=5 -4% predictor time; at N=6 the rolled form was
-  // 19% slower, so N=6 stays unrolled), and the double form of the
-  // 5-variable PDE at N=5, whose unrolled slices beside the closed first iteration exceed the 256
-  // registers of the two wavefronts per SIMD its LDS allows (with so many parameters that LDS does
-  // not hold all slices, they stay unrolled: a user's solver has no workspace).
-  static constexpr bool ROLLED = (B >= 7 && (IS_FP64 || B >= 8)) || V >= 9 || (!IS_FP64 && (B == 5 || B == 6)) ||
-                                 (IS_FP64 && B == 6 && V == 5 && (NQR == 0 || LDSK < 144));
+  // 19% slower, so N=6 stays unrolled).
+  // Double forms with fluxes up to N=5: rolled where the registers that unrolled
+  // slices take beside the closed first iteration (kUnrolled, fitted to the
+  // compiler's counts) are more than the wavefronts that LDS allows leave them,
+  // and with a non-conservative product besides, where the unrolled slices spill.
+  // 13,824 cells at N=4: flux and source 832 -> 597 us; 32,768 at N=3: flux and
+  // product of five variables 4170 -> 1380 us; where they fit, the unrolled
+  // slices are the faster ones (five variables at N=4, 13,824 cells: 574 us, rolled 599).
+  // Not without LDS for every slice, which would take a workspace (144 KB: a
+  // user's solver has none).
+  static constexpr int kUnrolled = 44 + (9 * B - 5) * V + 5 * (D - V) + (USE_SOURCE ? 10 * V : 0);
+  static constexpr long kLdsWaves = 160 * 1024 / (kOther + NQL * kSliceBytes) * (NT / kWave);  // per CU, of 4 SIMDs
+  static constexpr bool ROLLED_DOUBLE =
+      IS_FP64 && (NQR == 0 || LDSK < 144) && B >= 4 && B <= 6 &&
+      (!USE_FLUX ? B == 6 && V == 5 : (USE_NCP ? V >= 2 : kUnrolled > (kLdsWaves >= 6 ? 252 : 508)));
+  static constexpr bool ROLLED = (B >= 7 && (IS_FP64 || B >= 8)) || V >= 9 || (!IS_FP64 && (B == 5 || B == 6)) || ROLLED_DOUBLE;
   // 8+ waves per workgroup leave 256 registers per lane, no room for slices;
   // a rolled loop cannot index registers.
   static constexpr bool WSQ = NQR > 0 && (NT >= 8 * kWave || ROLLED);
@@ -163,7 +174,7 @@ __global__ __launch_bounds__(node_threads(B), (predictor_min_waves<B, PDE, TERMS
   constexpr bool USE_SRC_NCP = USE_SOURCE || USE_NCP;
   constexpr bool IS_FP64 = sizeof(T) == sizeof(double);
   constexpr int MAX_ITER = 2 * B;  // spaceTimePredictorNonlinear.cpph:85
-  using L = PredictorLayout<B, V, D, USE_NCP, T, LDSK, USE_FLUX>;
+  using L = PredictorLayout<B, V, D, USE_NCP, T, LDSK, USE_FLUX, USE_SOURCE>;
   constexpr int NQL = L::NQL, NQR = L::NQR, UNROLL_T = L::UNROLL_T;
   constexpr bool IN_PLACE = L::IN_PLACE;
   static_assert(!IN_PLACE || (NQL == B && B * V >= D), "the iterate's rows hold the epilogue's D");

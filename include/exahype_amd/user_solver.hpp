@@ -36,9 +36,9 @@ struct UserSolver {
   static_assert(ORDER >= 1 && ORDER <= 7, "orders 1..7");
   // The user route runs the predictor without a device workspace: every time
   // slice of the Picard iterate fits LDS or registers (orders up to 6 in FP64).
-  static constexpr bool USE_FLUX = (TERMS & kFlux) != 0;
-  static_assert(PredictorLayout<B, V, D, USE_NCP, double, 144, USE_FLUX>::ws_bytes == 0 &&
-                    PredictorLayout<B, V, D, USE_NCP, float, 144, USE_FLUX>::ws_bytes == 0,
+  static constexpr bool USE_FLUX = (TERMS & kFlux) != 0, USE_SOURCE = (TERMS & kSource) != 0;
+  static_assert(PredictorLayout<B, V, D, USE_NCP, double, 144, USE_FLUX, USE_SOURCE>::ws_bytes == 0 &&
+                    PredictorLayout<B, V, D, USE_NCP, float, 144, USE_FLUX, USE_SOURCE>::ws_bytes == 0,
                 "this order needs the predictor's device workspace, which user solvers do not have");
 
   static int predictor(const void* args, long ncells, int precision, void* stream) {

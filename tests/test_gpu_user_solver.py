@@ -178,6 +178,41 @@ def test_flux_free_user_pde_vs_oracle(exa, oracle, name, order, n, steps, npar):
         g.close()
 
 
+@pytest.mark.parametrize("order,other", [(3, "split_order3"), (4, "split_order4"), (5, "split_order5"),
+                                         (4, "source_order4")])
+@pytest.mark.parametrize("precision", [0, 1])
+def test_user_flux_with_product_or_source(exa, order, other, precision):
+    """Constant coefficients: half of a linear PDE as a flux and half as a
+    non-conservative product, or the flux beside a zero source, compute what the
+    flux alone does, but for rounding and the Picard iteration's end: face
+    fluxes are of the iterate before the last, states of the last, and in double
+    these differ by up to 1e-7 in the stopping norm.  States of size 1e6 put that
+    at 1e-13 of their scale a step, beside which 5 steps stay below 1e-12;
+    FP32-bulk, which stops at 1e-6 of the state's norm: 1e-6 relative L2.  These
+    forms run their time slices in rolled loops of their own."""
+    # (bound for iterations that end by the residual, as all do at the PDE's CFL
+    # number of 0.05; at 0.9 the limit of 2 (N + 1) iterations left 2e-11 of the scale)
+    print(f"case: user PDE waves {other} precision {precision}", flush=True)
+    n, D = (4, 3, 5), 5
+    cells = n[0] * n[1] * n[2]
+    luh = 1e6 * np.random.default_rng(order).uniform(-1, 1, (cells, (order + 1) ** 3, D))
+    out, its = [], []
+    for name in (f"order{order}", other):
+        g = exa.Grid.from_user_solver(getattr(exa.user_example(), f"exa_user_waves_{name}"), n, precision=precision)
+        g.upload(luh.ravel())
+        g.step(5)
+        out.append(g.solution().reshape(-1, D))
+        its.append(g.picard_iterations())
+        g.close()
+    assert max(its[0].max(), its[1].max()) < 2 * (order + 1)
+    a, b = out
+    if precision == 0:
+        assert np.array_equal(*its)
+        assert (np.abs(b - a).max(axis=0) <= TOL * np.abs(a).max(axis=0)).all()
+    else:
+        assert np.linalg.norm(b - a) <= 1e-6 * np.linalg.norm(a)
+
+
 def test_user_route_refusals(exa):
     L = exa.lib()
     b = exa.Grid(exa.euler_solver(3), 2)
