@@ -450,6 +450,8 @@ hipError_t launch_riemann(const SolverDesc& sd, const RiemannArgs& a, hipStream_
 
 hipError_t launch_update(const SolverDesc& sd, int mode, const UpdateArgs& a, long ncells, hipStream_t s) {
   if (ncells <= 0) return hipSuccess;
+  // linear solvers add their fluctuations in launch_corrector
+  if (sd.linear && (mode & kUpdSurface)) return hipErrorNotSupported;
   return dispatch_pde(sd, [&]<int B, class PDE>() -> hipError_t {
     const dim3 grid((unsigned)ncells), block(node_threads(B));
     if (sd.precision == kFP32Bulk) {

@@ -252,7 +252,8 @@ hipError_t launch_predictor_mfma(const SolverDesc& sd, const PredictorArgs& a, l
 // Cells per workspace chunk the host allocates for (bounds the workspace size).
 constexpr long kPredictorWsCells = 4096;
 hipError_t launch_riemann(const SolverDesc& sd, const RiemannArgs& a, hipStream_t s);
-// update_kernel modes: surface integral, solution update, write lduh back.
+// update_kernel modes: surface integral (the nonlinear one: refused for linear
+// solvers), solution update, write lduh back.
 enum : int { kUpdSurface = 1, kUpdUpdate = 2, kUpdWriteLduh = 4 };
 hipError_t launch_update(const SolverDesc& sd, int mode, const UpdateArgs& a, long ncells,
                          hipStream_t s);
