@@ -79,8 +79,11 @@ enum : int {
 // The launch_* functions below take the solver order (2..kLimMaxOrder, Euler,
 // FP64).  "all" launches cover every cell; the FV launches walk fv_list.
 bool limiter_supported(const SolverDesc& sd);
+// The per-step counters to zero, the FV list's length among them.
+hipError_t launch_lim_clear_flags(const LimArgs& a, hipStream_t s);
 // pst = st; flags cleared; FV list of cells with st >= A (its length is zero
-// before: launch_lim_update_status and launch_lim_init leave it so).
+// before: launch_lim_update_status and launch_lim_init leave it so; after a step
+// that did not get that far it takes launch_lim_clear_flags).
 hipError_t launch_lim_begin_step(const SolverDesc& sd, const LimArgs& a, hipStream_t s);
 // per interior face: merge the min/max face blocks (mergeSolutionMinMaxOnFace)
 hipError_t launch_lim_minmax_merge(const SolverDesc& sd, const LimArgs& a, const FaceDesc* faces, long nfaces,

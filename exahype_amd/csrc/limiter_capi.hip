@@ -85,6 +85,10 @@ struct exa_lgrid {
   exa::StepState* state = nullptr;
   void* ws = nullptr;
   long ws_cells = 0;
+  // a step began filling the FV list and its status kernel, which clears the
+  // list's length again, is not launched yet (true at a step's begin: a launch
+  // of the step before failed in between)
+  bool fv_list_open = false;
   bool profiling = false;
   bool fused_ts = false;      // fused time stepping (fuse-algorithmic-steps)
   double fused_weight = 0.9;  // fuse-algorithmic-steps-factor
@@ -216,7 +220,13 @@ hipError_t lstep(exa_lgrid* g) {
   const exa::LimArgs a = largs(g);
   const SolverDesc& sd = g->sd;
   hipStream_t s = g->stream;
-  hipError_t e = lstaged(g, EXA_STAGE_LIMITER, [&] { return exa::launch_lim_begin_step(sd, a, s); });
+  const bool broken = g->fv_list_open;
+  g->fv_list_open = true;
+  hipError_t e = lstaged(g, EXA_STAGE_LIMITER, [&] {
+    if (broken)
+      if (const hipError_t r = exa::launch_lim_clear_flags(a, s); r != hipSuccess) return r;
+    return exa::launch_lim_begin_step(sd, a, s);
+  });
   // Merging: DG Riemann problems unless both cells are FV-active
   // (LS:1575-1610); transmissive DG boundary faces need no work: Rusanov with
   // equal states returns the inner flux unchanged.
@@ -233,6 +243,7 @@ hipError_t lstep(exa_lgrid* g) {
     });
   if (e == hipSuccess) e = lstaged(g, EXA_STAGE_FV, [&] { return exa::launch_lim_fv_update(sd, a, false, s); });
   if (e == hipSuccess) e = lstaged(g, EXA_STAGE_UPDATE, [&] { return exa::launch_lim_update_status(sd, a, s); });
+  if (e == hipSuccess) g->fv_list_open = false;
   const int* irregular = g->flags + exa::kLimFlagIrregular;
   if (g->fused_ts) {
     // the cells' prediction with the predictor dt right after their update
@@ -397,6 +408,7 @@ static int lgrid_init_from_device(exa_lgrid* g, const double* d_lim_ic) {
   const exa::LimArgs a = largs(g);
   EXA_TRY(hipMemsetAsync(g->flags, 0, sizeof(int) * exa::kLimFlags, g->stream));  // new run: counters from zero
   EXA_TRY(exa::launch_lim_init(g->sd, a, d_lim_ic, g->stream));
+  g->fv_list_open = false;
   EXA_TRY(lstart(g));
   EXA_TRY(hipStreamSynchronize(g->stream));
   return EXA_OK;

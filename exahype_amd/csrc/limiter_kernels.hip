@@ -208,8 +208,9 @@ __device__ inline void load_tables(double* sUh2lim, double* sUh2lob, double* sLi
 // Step begin: flags cleared, pst = st, list of FV-active cells (st >= A).
 // ---------------------------------------------------------------------------
 // flags[0..2] and [4] are per step; flags[3] counts steps with an irregular
-// change.  The FV list's length is zero here: the status kernel of the previous
-// step cleared it behind its last reader.
+// change.  The FV list's length is zero at a step's begin: the status kernel of
+// the previous step cleared it behind its last reader (lim_clear_flags_kernel
+// where a launch failed before that kernel).
 __global__ void lim_clear_flags_kernel(int* flags) {
   if (threadIdx.x < kLimFlags && threadIdx.x != kLimFlagSteps) flags[threadIdx.x] = 0;
 }
@@ -846,8 +847,8 @@ __global__ __launch_bounds__(kStatusCells * kWave, 5) void lim_update_status_ker
 // ---------------------------------------------------------------------------
 // Irregular change: status spreading sweep (LimiterStatusSpreading.cpp +
 // LS:392-405) in -> out over interior faces; ensureRequiredLimiterPatchIsAllocated.
-// Sweep 0 also clears the dt slots and the FV list (they are rebuilt by the
-// rollback and the recomputation).
+// Sweep 0 also clears the dt slots (the recomputation fills them again; the FV
+// list is rebuilt from its own counter, which the step's begin cleared).
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void lim_spread_kernel(LimArgs a, const int* in, int* out, int sweep) {
   if (!a.flags[kLimFlagIrregular]) return;
@@ -1403,6 +1404,11 @@ bool limiter_supported(const SolverDesc& sd) {
          sd.order >= 2 && sd.order <= kLimMaxOrder && !sd.no_time_averaging;
 }
 
+hipError_t launch_lim_clear_flags(const LimArgs& a, hipStream_t s) {
+  hipLaunchKernelGGL(lim_clear_flags_kernel, dim3(1), dim3(64), 0, s, a.flags);
+  return hipGetLastError();
+}
+
 hipError_t launch_lim_begin_step(const SolverDesc& sd, const LimArgs& a, hipStream_t s) {
   (void)sd;
   hipLaunchKernelGGL(lim_begin_kernel, dim3(blocks256(a.ncells)), dim3(256), 0, s, a);
@@ -1494,8 +1500,9 @@ hipError_t launch_lim_recompute_finish(const SolverDesc& sd, const LimArgs& a, h
 }
 
 hipError_t launch_lim_init(const SolverDesc& sd, const LimArgs& a, const double* lim_ic, hipStream_t s) {
-  hipLaunchKernelGGL(lim_clear_flags_kernel, dim3(1), dim3(64), 0, s, a.flags);
-  hipError_t e = dispatch_lim(sd.order, [&]<int N>() -> hipError_t {
+  hipError_t e = launch_lim_clear_flags(a, s);
+  if (e != hipSuccess) return e;
+  e = dispatch_lim(sd.order, [&]<int N>() -> hipError_t {
     hipLaunchKernelGGL(lim_init_kernel<N>, dim3(a.ncells), dim3(kLimNT), 0, s, a);
     return hipGetLastError();
   });

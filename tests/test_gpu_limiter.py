@@ -9,6 +9,7 @@ blast problems (limiter status of every cell identical after every step, the
 same steps with an irregular change, dt to 1e-13, solution to 1e-12 of each
 variable's scale); at the full 81^3 size, size-independent invariants.
 """
+import ctypes
 import json
 import os
 
@@ -255,3 +256,33 @@ def test_more_patches_than_resident_workgroups_vs_oracle(exa, oracle, order, n, 
     for v in range(5):
         assert rel_max(sol[:, v], osol[:, v]) <= 1e-11, v
     g.close()
+
+
+def test_step_after_one_that_broke_off(exa):
+    """A step whose launches break off behind the one that lists the FV-active
+    cells (here because an earlier call of the program left an error with the
+    runtime, which the first launch reports) leaves the state where it was: the
+    step taken again continues as if nothing had happened, bit for bit."""
+    print("case: limiter step after one that broke off, N=2 7^3", flush=True)
+    maps = [line.split()[-1] for line in open("/proc/self/maps") if "libamdhip64" in line]
+    hip = ctypes.CDLL(maps[0])
+    nodes = np.array([0.1127016653792583, 0.5, 0.8872983346207417])
+    luh, lim_ic = blast_cells(2, 7, nodes=nodes, radius=0.3), blast_cells(2, 7, subcells=True, radius=0.3)
+    out = []
+    for breaks in (0, 3):
+        g = exa.LimitingGrid(exa.euler_solver(2), 7, boundary=exa.BC_TRANSMISSIVE)
+        g.upload(luh, lim_ic)
+        g.step(1)
+        g.synchronize()
+        for _ in range(breaks):
+            assert hip.hipSetDevice(1 << 20) != 0  # refused on the host; the runtime keeps the error
+            with pytest.raises(exa.ExaError):
+                g.step(1)
+        g.step(3)
+        st, irregular = g.status()
+        out.append((g.solution(), st, irregular))
+        g.close()
+    print(f"  FV-active cells {(out[0][1] >= 2).sum()}", flush=True)
+    assert (out[0][1] >= 2).sum() > 20
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
