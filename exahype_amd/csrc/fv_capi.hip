@@ -155,7 +155,7 @@ int muscl_setup(exa_fvgrid* g) {
   A((void**)&g->cur, nc);
   A((void**)&g->nbr, sizeof(int) * 6 * nc);
   A((void**)&g->fv_list, sizeof(int) * nc);
-  A((void**)&g->flags, sizeof(int) * 3);
+  A((void**)&g->flags, exa::kLimFlagBytes);
   A((void**)&g->step, sizeof(exa::StepState));
   if (e != hipSuccess) return from_hip(e);
   EXA_TRY(hipMemsetAsync(g->lim, 0, sizeof(double) * patch * 2 * nc, g->stream));
@@ -180,7 +180,8 @@ int muscl_setup(exa_fvgrid* g) {
       nbr[6 * c + f] = (int)(((long)kk * g->ny + jj) * g->nx + ii);
     }
   }
-  const int flags[3] = {0, (int)nc, 0};
+  int flags[exa::kLimFlags] = {};
+  flags[exa::kLimFlagFvCount] = (int)nc;
   EXA_TRY(hipMemcpyAsync(g->nbr, nbr.data(), sizeof(int) * nbr.size(), hipMemcpyHostToDevice, g->stream));
   EXA_TRY(hipMemcpyAsync(g->fv_list, list.data(), sizeof(int) * nc, hipMemcpyHostToDevice, g->stream));
   EXA_TRY(hipMemcpyAsync(g->flags, flags, sizeof(flags), hipMemcpyHostToDevice, g->stream));

@@ -75,6 +75,7 @@ enum : int {
   kLimFlagFvAgain = 4,
   kLimFlags = 5
 };
+constexpr size_t kLimFlagBytes = sizeof(int) * kLimFlags;  // of every LimArgs::flags
 
 // The launch_* functions below take the solver order (2..kLimMaxOrder, Euler,
 // FP64).  "all" launches cover every cell; the FV launches walk fv_list.

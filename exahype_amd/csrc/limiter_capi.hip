@@ -343,7 +343,7 @@ extern "C" int exa_lgrid_create(const exa_solver* s, int nx, int ny, int nz, con
   A((void**)&g->st2, sizeof(int) * ncells);
   A((void**)&g->itc, sizeof(int) * ncells);
   A((void**)&g->nbr, sizeof(int) * ncells * 6);
-  A((void**)&g->flags, sizeof(int) * exa::kLimFlags);
+  A((void**)&g->flags, exa::kLimFlagBytes);
   A((void**)&g->fv_list, sizeof(int) * ncells);
   A((void**)&g->rc_list, sizeof(int) * ncells);
   A((void**)&g->loc_mm, sizeof(double) * ncells * 10);
@@ -356,7 +356,7 @@ extern "C" int exa_lgrid_create(const exa_solver* s, int nx, int ny, int nz, con
   }
   // patch edges and corners must read zero forever (FiniteVolumesSolver.cpp:477-481)
   if (e == hipSuccess) e = hipMemsetAsync(g->lim, 0, sizeof(double) * ncells * 2 * patch, g->stream);
-  if (e == hipSuccess) e = hipMemsetAsync(g->flags, 0, sizeof(int) * exa::kLimFlags, g->stream);
+  if (e == hipSuccess) e = hipMemsetAsync(g->flags, 0, exa::kLimFlagBytes, g->stream);
   if (e == hipSuccess) e = hipMemcpyAsync(g->d_dx, g->dx, sizeof(double) * 3, hipMemcpyHostToDevice, g->stream);
   // neighbours and the interior face list (each face once, owned by its left cell)
   std::vector<int> nbr(ncells * 6);
@@ -406,7 +406,7 @@ extern "C" long exa_lgrid_num_cells(const exa_lgrid* g) { return g ? g->ncells :
 
 static int lgrid_init_from_device(exa_lgrid* g, const double* d_lim_ic) {
   const exa::LimArgs a = largs(g);
-  EXA_TRY(hipMemsetAsync(g->flags, 0, sizeof(int) * exa::kLimFlags, g->stream));  // new run: counters from zero
+  EXA_TRY(hipMemsetAsync(g->flags, 0, exa::kLimFlagBytes, g->stream));  // new run: counters from zero
   EXA_TRY(exa::launch_lim_init(g->sd, a, d_lim_ic, g->stream));
   g->fv_list_open = false;
   EXA_TRY(lstart(g));
@@ -668,7 +668,7 @@ extern "C" int exa_musclhancock_solution_update(const exa_solver* s, double* luh
   EXA_TRY(d_mm.alloc(sizeof(double) * 10));
   EXA_TRY(d_cur.alloc(1));
   EXA_TRY(d_list.alloc(sizeof(int)));
-  EXA_TRY(d_flags.alloc(sizeof(int) * exa::kLimFlags));
+  EXA_TRY(d_flags.alloc(exa::kLimFlagBytes));
   EXA_TRY(d_dx.alloc(sizeof(double) * 3));
   EXA_TRY(d_state.alloc(sizeof(exa::StepState)));
   EXA_TRY(d_dtmax.alloc(sizeof(unsigned long long)));
@@ -677,7 +677,7 @@ extern "C" int exa_musclhancock_solution_update(const exa_solver* s, double* luh
   EXA_TRY(hipMemcpy(d_lim.p, luh, sizeof(double) * patch, hipMemcpyHostToDevice));
   EXA_TRY(hipMemcpy(d_lim.d() + patch, luh_new, sizeof(double) * patch, hipMemcpyHostToDevice));
   EXA_TRY(hipMemset(d_cur.p, 0, 1));
-  EXA_TRY(hipMemset(d_flags.p, 0, sizeof(int) * exa::kLimFlags));
+  EXA_TRY(hipMemset(d_flags.p, 0, exa::kLimFlagBytes));
   EXA_TRY(hipMemcpy(d_dx.p, dx, sizeof(double) * 3, hipMemcpyHostToDevice));
   EXA_TRY(hipMemcpy(d_state.p, &dt, sizeof(double), hipMemcpyHostToDevice));  // StepState::dt is first
   exa::LimArgs a{};

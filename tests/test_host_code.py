@@ -1,5 +1,6 @@
 """Host-side C++ of the library, in small programs built and run without a GPU."""
 import os
+import re
 import subprocess
 
 import pytest
@@ -49,3 +50,16 @@ int main() {
 }
 """, *library)
     assert res.returncode == 0, res.stderr
+
+
+def test_limiter_counters_are_allocated_whole():
+    """Every owner of the limiter kernels' counters allocates and clears all of
+    them, whichever its calls read today."""
+    owners = 0
+    for name in sorted(os.listdir(os.path.join(build.HERE, "csrc"))):
+        text = open(os.path.join(build.HERE, "csrc", name)).read()
+        for stmt in re.findall(r"[^;{}]*flags[^;{}]*;", text):
+            if re.search(r"\b(hipMalloc|A\(|alloc\(|hipMemset)", stmt) and not re.search(r"CreateWithFlags", stmt):
+                assert "kLimFlagBytes" in stmt, (name, stmt.strip())
+                owners += 1
+    assert owners >= 3
