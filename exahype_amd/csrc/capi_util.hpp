@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 #include <cstring>
 #include <memory>
@@ -80,19 +81,20 @@ class CallBuffers {
   }
   // Allocates, lays the parts out and copies the inputs up.
   hipError_t up() {
+    if (full_) return hipErrorInvalidValue;
     size_t end = 0;
     for (int k = 0; k < kKinds; ++k) {
       begin_[k] = end;
       for (int i = 0; i < n_; ++i)
         if (part_[i].kind == k) {
           part_[i].offset = end;
-          end += (part_[i].bytes + 255) / 256 * 256;
+          end += (std::max<size_t>(part_[i].bytes, 8) + 255) / 256 * 256;
         }
     }
     begin_[kKinds] = end;
     if (hipError_t e = mem_.alloc(end); e != hipSuccess) return e;
-    const size_t lo = begin_[kInOut], hi = begin_[kScratch];  // kInOut and kIn
-    if (end <= kPackBytes) host_.reset(new (std::nothrow) char[end]);
+    const size_t lo = begin_[kInOut], hi = begin_[kScratch];  // kInOut and kIn; scratch is not packed
+    if (hi <= kPackBytes) host_.reset(new (std::nothrow) char[hi]);
     for (int i = 0; i < n_; ++i) {
       const Part& p = part_[i];
       if (p.kind != kIn && p.kind != kInOut) continue;
@@ -143,12 +145,18 @@ class CallBuffers {
     Kind kind;
   };
   int add(const void* from, void* to, size_t bytes, Kind kind) {
-    part_[n_] = {from, to, bytes ? bytes : 8, 0, kind};
+    if (n_ == kParts) {  // reported by up()
+      full_ = true;
+      return n_ - 1;
+    }
+    part_[n_] = {from, to, bytes, 0, kind};
     return n_++;
   }
   void* at(int i) const { return static_cast<char*>(mem_.p) + part_[i].offset; }
-  Part part_[16];
+  static constexpr int kParts = 16;
+  Part part_[kParts];
   int n_ = 0;
+  bool full_ = false;
   size_t begin_[kKinds + 1] = {};
   DevBuf mem_;
   std::unique_ptr<char[]> host_;

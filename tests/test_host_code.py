@@ -63,3 +63,73 @@ def test_limiter_counters_are_allocated_whole():
                 assert "kLimFlagBytes" in stmt, (name, stmt.strip())
                 owners += 1
     assert owners >= 3
+
+
+# the runtime's calls as host functions that count: device memory is host memory
+FAKE_HIP = r"""
+#include "capi_util.hpp"
+#include <cstdio>
+#include <cstdlib>
+#include <numeric>
+#include <vector>
+static int ups, downs, sets;
+extern "C" {
+hipError_t hipMalloc(void** p, size_t n) { *p = std::malloc(n); std::memset(*p, 0x5a, n); return hipSuccess; }
+hipError_t hipFree(void* p) { std::free(p); return hipSuccess; }
+hipError_t hipMemset(void* p, int v, size_t n) { ++sets; std::memset(p, v, n); return hipSuccess; }
+hipError_t hipDeviceSynchronize() { return hipSuccess; }
+hipError_t hipMemcpy(void* to, const void* from, size_t n, hipMemcpyKind k) {
+  ++(k == hipMemcpyHostToDevice ? ups : downs);
+  std::memcpy(to, from, n);
+  return hipSuccess;
+}
+}
+#define CHECK(c) if (!(c)) { std::printf("line %d: %s\n", __LINE__, #c); return 1; }
+"""
+
+
+@pytest.mark.parametrize("scratch,inputs,packed", [(0, 4096, True), (1 << 19, 900 << 10, True), (1 << 21, 64, True),
+                                                   (0, 1 << 20, False), (64, 2 << 20, False)])
+def test_buffers_of_a_call(tmp_path, scratch, inputs, packed):
+    """One copy each way up to 1 MiB of inputs and outputs, whatever the scratch;
+    array by array above.  Inputs, outputs, both, cleared and empty parts."""
+    res = _run(tmp_path, FAKE_HIP + r"""
+int main() {
+  const size_t n = %d / 8, m = 256;
+  std::vector<double> in(n), io(m, 2.0), out(m), zero(m, -1.0);
+  std::iota(in.begin(), in.end(), 1.0);
+  CallBuffers b;
+  const int i_in = b.in(in.data(), n * 8), i_out = b.out(out.data(), m * 8), i_none = b.in(nullptr, 0);
+  const int i_io = b.inout(io.data(), io.data(), m * 8), i_zero = b.out(zero.data(), m * 8, true);
+  const int i_scratch = b.scratch(%d), i_z2 = b.zeroed(m * 8);
+  CHECK(b.up() == hipSuccess);
+  CHECK(i_none != i_in && i_scratch != i_z2);
+  for (size_t k = 0; k < m; ++k) {  // the call's kernel
+    CHECK(b.d(i_zero)[k] == 0.0 && b.d(i_z2)[k] == 0.0);
+    b.d(i_out)[k] = b.d(i_in)[k %% n] + b.d(i_io)[k];
+    b.d(i_io)[k] *= 3.0;
+  }
+  std::memset(b.d(i_scratch), 0, %d);
+  CHECK(b.down() == hipSuccess);
+  for (size_t k = 0; k < m; ++k) CHECK(out[k] == in[k %% n] + 2.0 && io[k] == 6.0 && zero[k] == 0.0);
+  std::printf("up %%d down %%d set %%d\n", ups, downs, sets);
+  return 0;
+}
+""" % (inputs, scratch, scratch))
+    assert res.returncode == 0, res.stdout
+    assert res.stdout.split() == (["up", "1", "down", "1", "set", "0"] if packed else
+                                  ["up", "2", "down", "3", "set", "3"])
+
+
+def test_buffers_of_a_call_too_many_parts(tmp_path):
+    """More parts than a call can have are refused, not written past the table."""
+    res = _run(tmp_path, FAKE_HIP + r"""
+int main() {
+  struct { CallBuffers b; } x;
+  double v[64] = {};
+  for (int k = 0; k < 64; ++k) CHECK(x.b.in(v + k, 8) < 16);
+  CHECK(x.b.up() == hipErrorInvalidValue);
+  return 0;
+}
+""")
+    assert res.returncode == 0, res.stdout + res.stderr
