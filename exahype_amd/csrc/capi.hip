@@ -198,21 +198,22 @@ extern "C" int exa_riemann_solver_nonlinear(const exa_solver* s, double* FL, dou
   if (!to_desc(s, &sd) || !FL || !FR || !QL || !QR || direction < 0 || direction > 2) return EXA_E_INVALID;
   if (sd.linear || !exa::supported(sd) || sd.precision != exa::kFP64) return EXA_E_UNSUPPORTED;
   const Sizes z(sd);
-    // One cell's face blocks, with the left state at 2d+1 and the right one at 2d
-  // (as if the cell were its own neighbour).
+  // One cell's face blocks, with the left state at 2d+1 and the right one at 2d
+  // (as if the cell were its own neighbour).  On the heap: up to 21 KB each, and a
+  // caller's thread may have a small stack.
   const long qf = z.B2 * z.D, ff = z.B2 * z.V;
-  constexpr long kMost = 64 * 16;  // B^2 D of every compiled solver is below
-  if (qf > kMost) return EXA_E_UNSUPPORTED;
-  double q[6 * kMost] = {}, F[6 * kMost] = {};
-  double *const q_right = q + 2 * direction * qf, *const q_left = q_right + qf;
-  double *const F_right = F + 2 * direction * ff, *const F_left = F_right + ff;
+  const std::unique_ptr<double[]> q(new (std::nothrow) double[6 * qf]()), F(new (std::nothrow) double[6 * ff]());
+  if (!q || !F) return EXA_E_NOMEM;
+  double *const q_right = q.get() + 2 * direction * qf, *const q_left = q_right + qf;
+  double *const F_right = F.get() + 2 * direction * ff, *const F_left = F_right + ff;
   std::copy_n(QL, qf, q_left);
   std::copy_n(QR, qf, q_right);
   std::copy_n(FL, ff, F_left);
   std::copy_n(FR, ff, F_right);
   const FaceDesc f{0, 0, direction, 0};
   CallBuffers buf;
-  const int b_q = buf.in(q, sizeof(double) * 6 * qf), b_f = buf.inout(F, F, sizeof(double) * 6 * ff);
+  const int b_q = buf.in(q.get(), sizeof(double) * 6 * qf);
+  const int b_f = buf.inout(F.get(), F.get(), sizeof(double) * 6 * ff);
   const int b_face = buf.in(&f, sizeof(f));
   EXA_TRY(buf.up());
   exa::RiemannArgs a{buf.as<const FaceDesc>(b_face), 1, buf.d(b_q), buf.d(b_f)};
@@ -361,7 +362,8 @@ extern "C" int exa_riemann_solver_linear(const exa_solver* s, double* FL, double
   sd.linear = 1;
   if (!exa::linear_supported(sd)) return EXA_E_UNSUPPORTED;
   const Sizes z(sd);
-    DevBuf d_qb, d_fb, d_face;
+  // Two cells: cell 0 owns face 2d+1 (left state), cell 1 owns face 2d (right state).
+  DevBuf d_qb, d_fb, d_face;
   const long qf = z.B2 * z.D, ff = z.B2 * z.V;
   EXA_TRY(d_qb.alloc(sizeof(double) * 2 * 6 * qf));
   EXA_TRY(d_fb.alloc(sizeof(double) * 2 * 6 * ff));

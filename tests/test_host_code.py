@@ -133,3 +133,37 @@ int main() {
 }
 """)
     assert res.returncode == 0, res.stdout + res.stderr
+
+
+def test_riemann_call_on_a_small_stack(tmp_path, library):
+    """The single-face Riemann call runs on a thread with 96 KiB of stack (its
+    status is that of the device, absent or not)."""
+    res = _run(tmp_path, r"""
+#include "exahype_amd.h"
+#include <cstdio>
+#include <pthread.h>
+static exa_solver s;
+static double FL[320], FR[320], QL[384], QR[384];
+static void* call(void* status) {
+  *static_cast<int*>(status) = exa_riemann_solver_nonlinear(&s, FL, FR, QL, QR, 0.1, 1);
+  return nullptr;
+}
+int main() {
+  s.pde = EXA_PDE_EULER;
+  s.order = 3;
+  s.num_variables = 5;
+  s.terms = EXA_TERM_FLUX;
+  s.cfl = 0.9;
+  for (int k = 0; k < 80; k += 5) QL[k] = QR[k] = 1.0, QL[k + 4] = QR[k + 4] = 2.5;
+  int here = -1, there = -2;
+  call(&here);  // the runtime starts on this thread
+  pthread_attr_t a;
+  pthread_t t;
+  pthread_attr_init(&a);
+  if (pthread_attr_setstacksize(&a, 96 << 10) != 0 || pthread_create(&t, &a, call, &there) != 0) return 2;
+  pthread_join(t, nullptr);
+  std::printf("%d %d\n", here, there);
+  return here == there && here != EXA_E_INVALID && here != EXA_E_UNSUPPORTED ? 0 : 1;
+}
+""", "-lpthread", *library)
+    assert res.returncode == 0, (res.returncode, res.stdout, res.stderr)
