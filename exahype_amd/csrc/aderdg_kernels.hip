@@ -332,6 +332,7 @@ hipError_t launch_predictor(const SolverDesc& sd, bool export_temps, const Predi
   if (ws > 0 && (a.ws == nullptr || a.ws_cells <= 0)) return hipErrorInvalidValue;
   const long chunk = ws > 0 ? a.ws_cells : ncells;
   return dispatch_pde(sd, [&]<int B, class PDE>() -> hipError_t {
+    constexpr int kLds64 = PDE::P == 0 ? 64 : 144;  // the 64 KB variant is compiled without parameters only
     // chunks of at most ws_cells cells share the workspace (stream order)
     for (long c0 = 0; c0 < ncells; c0 += chunk) {
       PredictorArgs ac = a;
@@ -354,13 +355,13 @@ hipError_t launch_predictor(const SolverDesc& sd, bool export_temps, const Predi
         }
       } else if (sd.precision == kFP32Bulk) {
         if (sd.terms != kFlux) return hipErrorNotSupported;
-        if (a.variant == kPredictorValu64 && PDE::P == 0)
-          hipLaunchKernelGGL((predictor_kernel<B, PDE, kFlux, false, float, 64>), grid, block, 0, s, ac);
+        if (a.variant == kPredictorValu64)
+          hipLaunchKernelGGL((predictor_kernel<B, PDE, kFlux, false, float, kLds64>), grid, block, 0, s, ac);
         else
           hipLaunchKernelGGL((predictor_kernel<B, PDE, kFlux, false, float>), grid, block, 0, s, ac);
       } else if (sd.terms == kFlux) {
-        if (a.variant == kPredictorValu64 && PDE::P == 0 && !export_temps)
-          hipLaunchKernelGGL((predictor_kernel<B, PDE, kFlux, false, double, 64>), grid, block, 0, s, ac);
+        if (a.variant == kPredictorValu64 && !export_temps)
+          hipLaunchKernelGGL((predictor_kernel<B, PDE, kFlux, false, double, kLds64>), grid, block, 0, s, ac);
         else if (export_temps)
           hipLaunchKernelGGL((predictor_kernel<B, PDE, kFlux, true, double>), grid, block, 0, s, ac);
         else

@@ -29,18 +29,19 @@ namespace exa {
 // cells, N=7 1.66 -> 1.71 ms for 20,000; N=3 double 0.527 -> 0.60 ms for 30,000).
 template <int B, class PDE>
 struct WaveLayout {
-  static constexpr int V = PDE::V, P = PDE::P, D = V + P;
+  static_assert(PDE::P == 0, "the iterate's registers hold variables only");
+  static constexpr int V = PDE::V;
   static constexpr int B3 = B * B * B;
   static constexpr int NT = B * kWave;
   static constexpr int C = (B3 + kWave - 1) / kWave;  // nodes per lane
   static constexpr int ROWS = B * V;                  // V rows per slice
-  static constexpr int EROWS = 3 * V > D ? 3 * V : D;  // sums over the slices (epilogue, first iteration)
+  static constexpr int EROWS = 3 * V;                 // sums over the slices (epilogue, first iteration)
 };
 
 template <int B, class PDE, typename T>
 __global__ __launch_bounds__(B* kWave, (sizeof(T) == sizeof(float) ? 3 : 2)) void predictor_wave_kernel(PredictorArgs a) {
   using L = WaveLayout<B, PDE>;
-  constexpr int V = L::V, P = L::P, D = L::D;
+  constexpr int V = L::V;
   constexpr int N = B - 1, B2 = B * B, B3 = L::B3, NT = L::NT, C = L::C;
   constexpr bool IS_FP64 = sizeof(T) == sizeof(double);
   constexpr int MAX_ITER = 2 * B;  // spaceTimePredictorNonlinear.cpph:85
@@ -63,7 +64,7 @@ __global__ __launch_bounds__(B* kWave, (sizeof(T) == sizeof(float) ? 3 : 2)) voi
   T gd[3];  // dt / dx_d
 #pragma unroll
   for (int d = 0; d < 3; ++d) gd[d] = wave_uniform(dt * (T(1.0) / T(dxp[d])));
-  const double* const luh = a.luh + cell * (size_t)(B3 * D);
+  const double* const luh = a.luh + cell * (size_t)(B3 * V);
   T* const sG = sS + t * (V * B3);
   // node c of this lane; surplus nodes repeat the last one and store nothing
   auto node_of = [&](int c) __device__ { return (c + 1) * kWave <= B3 || lane + c * kWave < B3 ? lane + c * kWave : B3 - 1; };
@@ -121,16 +122,15 @@ __global__ __launch_bounds__(B* kWave, (sizeof(T) == sizeof(float) ? 3 : 2)) voi
   };
 
   T qi[C][V];           // lQi^k(t)
-  T par[P > 0 ? C : 1][P > 0 ? P : 1];
   int iters = MAX_ITER;
 
   // First iteration: every slice of the initial iterate equals luh, so one
   // evaluation R = dt sum_d dF_d/dx_d of luh serves all slices:
   // lQi^1(l) = a_l luh - b_l R.
   for (int n = tid; n < B3; n += NT) {
-    T Q[D], F[3][V];
+    T Q[V], F[3][V];
 #pragma unroll
-    for (int m = 0; m < D; ++m) Q[m] = T(luh[(size_t)n * D + m]);
+    for (int m = 0; m < V; ++m) Q[m] = T(luh[(size_t)n * V + m]);
     PDE::flux(Q, F);
 #pragma unroll
     for (int d = 0; d < 3; ++d)
@@ -150,13 +150,11 @@ __global__ __launch_bounds__(B* kWave, (sizeof(T) == sizeof(float) ? 3 : 2)) voi
       const int n = node_of(c);
 #pragma unroll
       for (int m = 0; m < V; ++m) {
-        const T q = T(luh[(size_t)n * D + m]);
+        const T q = T(luh[(size_t)n * V + m]);
         const T R = gd[0] * sE[m * B3 + n] + gd[1] * sE[(V + m) * B3 + n] + gd[2] * sE[(2 * V + m) * B3 + n];
         qi[c][m] = q;
         qn[c][m] = al * q - bl * R;
       }
-#pragma unroll
-      for (int m = 0; m < P; ++m) par[c][m] = T(luh[(size_t)n * D + V + m]);
       __builtin_amdgcn_sched_barrier(0);
     }
   }
@@ -212,9 +210,9 @@ __global__ __launch_bounds__(B* kWave, (sizeof(T) == sizeof(float) ? 3 : 2)) voi
     auto direction = [&]<int DIR>() __device__ __attribute__((always_inline)) {
 #pragma unroll
       for (int c = 0; c < C; ++c) {
-        T Q[D], F[3][V];
+        T Q[V], F[3][V];
 #pragma unroll
-        for (int m = 0; m < D; ++m) Q[m] = m < V ? qi[c][m < V ? m : 0] : par[P > 0 ? c : 0][m >= V ? m - V : 0];
+        for (int m = 0; m < V; ++m) Q[m] = qi[c][m];
 #pragma unroll
         for (int m = 0; m < V; ++m) asm volatile("" : "+v"(Q[m]));
         PDE::flux(Q, F);
@@ -280,8 +278,7 @@ __global__ __launch_bounds__(B* kWave, (sizeof(T) == sizeof(float) ? 3 : 2)) voi
 
   // ---- epilogue: time average, extrapolation, volume integral ----
   asm volatile("" : "+v"(tid));  // its index arithmetic stays here: nothing of it is held across the iterations
-  const size_t cQb = cell * (size_t)(6 * B2 * D);
-  const size_t cFb = cell * (size_t)(6 * B2 * V);
+  const size_t cb = cell * (size_t)(6 * B2 * V);
   T* const out_lduh = static_cast<T*>(a.lduh);
   T* const out_lQhbnd = static_cast<T*>(a.lQhbnd);
   T* const out_lFhbnd = static_cast<T*>(a.lFhbnd);
@@ -332,28 +329,18 @@ __global__ __launch_bounds__(B* kWave, (sizeof(T) == sizeof(float) ? 3 : 2)) voi
 #pragma unroll
       for (int m = 0; m < V; ++m) sG[m * B3 + node_of(c)] = wt * qn[c][m];
     }
-  if constexpr (P > 0) {
-    if (t == 0) {
-#pragma unroll
-      for (int c = 0; c < C; ++c)
-        if (owns(c)) {
-#pragma unroll
-          for (int m = 0; m < P; ++m) sE[(V + m) * B3 + node_of(c)] = par[c][m];
-        }
-    }
-  }
   add_slices(sE);
-  extrapolate.template operator()<0, D>(sE, out_lQhbnd, cQb);
-  extrapolate.template operator()<1, D>(sE, out_lQhbnd, cQb);
-  extrapolate.template operator()<2, D>(sE, out_lQhbnd, cQb);
+  extrapolate.template operator()<0, V>(sE, out_lQhbnd, cb);
+  extrapolate.template operator()<1, V>(sE, out_lQhbnd, cb);
+  extrapolate.template operator()<2, V>(sE, out_lQhbnd, cb);
   // Time-averaged fluxes of the last evaluation, i.e. of lQi^k = qi (:96-122
   // vs :306, :367-396): lFhi_d = sum_t w_t F_d(lQi^k(t)).
   auto average = [&]<int DIR>() __device__ __attribute__((always_inline)) {
 #pragma unroll
     for (int c = 0; c < C; ++c) {
-      T Q[D], F[3][V];
+      T Q[V], F[3][V];
 #pragma unroll
-      for (int m = 0; m < D; ++m) Q[m] = m < V ? qi[c][m < V ? m : 0] : par[P > 0 ? c : 0][m >= V ? m - V : 0];
+      for (int m = 0; m < V; ++m) Q[m] = qi[c][m];
       PDE::flux(Q, F);
       if (owns(c)) {
 #pragma unroll
@@ -366,9 +353,9 @@ __global__ __launch_bounds__(B* kWave, (sizeof(T) == sizeof(float) ? 3 : 2)) voi
   average.template operator()<0>();
   average.template operator()<1>();
   average.template operator()<2>();
-  extrapolate.template operator()<0, V>(sE, out_lFhbnd, cFb);
-  extrapolate.template operator()<1, V>(sE + V * B3, out_lFhbnd, cFb);
-  extrapolate.template operator()<2, V>(sE + 2 * V * B3, out_lFhbnd, cFb);
+  extrapolate.template operator()<0, V>(sE, out_lFhbnd, cb);
+  extrapolate.template operator()<1, V>(sE + V * B3, out_lFhbnd, cb);
+  extrapolate.template operator()<2, V>(sE + 2 * V * B3, out_lFhbnd, cb);
   if (a.iters && tid == 0) a.iters[cell] = iters;
   if (!out_lduh) return;
   // volume integral (volumeIntegralNonlinear.cpph:136-225): the directional
