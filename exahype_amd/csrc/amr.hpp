@@ -11,9 +11,8 @@ constexpr int kAmrMaxLevelDelta = 6;  // 3^6 = 729 subintervals per direction
 // A batch of transfers between blocks of B^NDIM nodes x nv values (volumes:
 // (z,y,x,var); faces: (b,a,var)).  items: 5 ints per transfer (destination
 // block, source block, subinterval index per direction in [0, 3^level_delta);
-// faces use the first two).  Prolongation: one wavefront per item, the
-// destination overwritten.  Restriction: one workgroup per destination k over
-// items [ptr[k], ptr[k+1]), which must share one destination block; their
+// faces use the first two).  Prolongation: the destination overwritten.
+// Restriction: one workgroup per destination k over items [ptr[k], ptr[k+1]), which must share one destination block; their
 // restricted blocks are added to it in list order.  Items with an index out of
 // range (or a mismatched destination) are skipped and set *error.  Every
 // destination block may appear once per launch (one item of a prolongation,

@@ -229,3 +229,94 @@ def test_batches_uneven_ranges_vs_oracle(exa, oracle, order, nv, children):
     for it in items:
         acc[it[1]] = oracle.volume_unknowns_restriction(os_, acc[it[1]], fine_in[it[0]], 0, 1, it[2:])
     assert _rel(d_acc.get(), acc) <= 1e-12
+
+
+def _any_solver(exa, oracle, order, nv):
+    return (exa.Solver(exa.PDE_EULER, order, nv, 0, exa.TERM_FLUX, 0, 0.9, exa.PRECISION_FP64, 0),
+            oracle.make_solver(order, nvar=nv, npar=0))
+
+
+# (order, values per node, transfers, levels): both sides of the lines between a
+# thread per value, a workgroup and a wavefront per transfer
+PROLONGATIONS = [(1, 1, 7, 3), (3, 4, 2100, 1), (2, 10, 2048, 1), (2, 10, 2049, 2), (3, 8, 1153, 1), (4, 8, 1152, 1),
+                 (4, 8, 1153, 1), (3, 17, 500, 2), (5, 5, 512, 1), (5, 5, 513, 1), (5, 9, 513, 1), (5, 12, 600, 1),
+                 (5, 12, 3, 2)]
+
+
+@pytest.mark.parametrize("order,nv,count,levels", PROLONGATIONS)
+def test_prolongation_forms(exa, oracle, order, nv, count, levels):
+    """One long list against the same transfers in lists of 50, which take other
+    forms of the kernel with the same sums in the same order (1e-14), and single
+    transfers against the oracle."""
+    print(f"case: AMR prolongation forms N={order} nv={nv} {count} transfers {levels} levels", flush=True)
+    rng = np.random.default_rng(order * 1000 + nv + count)
+    s, os_ = _any_solver(exa, oracle, order, nv)
+    blk, r = (order + 1) ** 3 * nv, 3 ** levels
+    coarse = rng.standard_normal((5, blk))
+    items = np.column_stack([rng.permutation(count), rng.integers(0, 5, count),
+                             rng.integers(0, r, (count, 3))]).astype(np.int32)
+    d_c, d_f = exa.DeviceArray(coarse), exa.DeviceArray(np.zeros((count, blk)))
+    exa.volume_prolongation_batch(s, d_f, d_c, exa.DeviceArray(items), levels)
+    fine = d_f.get()
+    d_g = exa.DeviceArray(np.zeros((count, blk)))
+    for k in range(0, count, 50):
+        exa.volume_prolongation_batch(s, d_g, d_c, exa.DeviceArray(items[k:k + 50]), levels)
+    assert _rel(fine, d_g.get()) <= 1e-14
+    for it in items[:: max(1, count // 5)]:
+        ref = oracle.volume_unknowns_prolongation(os_, coarse[it[1]], 0, levels, it[2:])
+        assert _rel(fine[it[0]], ref) <= 1e-12
+
+
+@pytest.mark.parametrize("order,nv,count", [(2, 3, 40), (4, 8, 40), (4, 12, 40), (4, 8, 1300)])
+def test_prolongation_forms_report_bad_items(exa, oracle, order, nv, count):
+    """Every form skips an item out of range and writes a block named twice once,
+    and the call fails."""
+    print(f"case: AMR prolongation bad items N={order} nv={nv} {count} transfers", flush=True)
+    rng = np.random.default_rng(count + nv)
+    s, os_ = _any_solver(exa, oracle, order, nv)
+    blk = (order + 1) ** 3 * nv
+    coarse = rng.standard_normal((2, blk))
+    items = np.column_stack([np.arange(count), rng.integers(0, 2, count), rng.integers(0, 3, (count, 3))])
+    items = items.astype(np.int32)
+    items[7, 0] = count  # no such block
+    items[9, 3] = 3      # no such subcell
+    items[20, 0] = 19    # block 19 twice
+    d_c, d_f = exa.DeviceArray(coarse), exa.DeviceArray(np.zeros((count, blk)))
+    with pytest.raises(exa.ExaError):
+        exa.volume_prolongation_batch(s, d_f, d_c, exa.DeviceArray(items), 1)
+    fine = d_f.get()
+    assert not fine[[7, 9, 20]].any()
+    ref = [oracle.volume_unknowns_prolongation(os_, coarse[it[1]], 0, 1, it[2:]) for it in items[[18, 19, 20]]]
+    assert _rel(fine[18], ref[0]) <= 1e-12
+    assert min(_rel(fine[19], ref[1]), _rel(fine[19], ref[2])) <= 1e-12
+
+
+@pytest.mark.parametrize("order,nv,children,levels", [(4, 13, (9, 0, 4, 1), 1), (5, 8, (1, 5, 0, 27), 1),
+                                                      (5, 12, (3, 0, 6, 1), 2), (3, 25, (2, 5, 1, 3), 1)])
+def test_restriction_of_large_blocks_vs_oracle(exa, oracle, order, nv, children, levels):
+    """Blocks of which 64 KiB hold four and a destination, and of which they do
+    not (a workgroup per transfer); an item out of range is skipped."""
+    print(f"case: AMR restriction N={order} nv={nv} children={children} levels={levels}", flush=True)
+    rng = np.random.default_rng(order + nv)
+    s, os_ = _any_solver(exa, oracle, order, nv)
+    blk, n = (order + 1) ** 3 * nv, sum(children)
+    items = np.column_stack([np.repeat(np.arange(len(children)), children), rng.permutation(n),
+                             rng.integers(0, 3 ** levels, (n, 3))]).astype(np.int32)
+    ptr = np.concatenate([[0], np.cumsum(children)]).astype(np.int32)
+    coarse, fine = rng.standard_normal((len(children), blk)), rng.standard_normal((n, blk))
+    for bad in (None, 1):
+        it_run = items.copy()
+        if bad is not None:
+            it_run[bad, 1] = n  # no such block
+        d_acc = exa.DeviceArray(coarse)
+        call = (s, d_acc, exa.DeviceArray(fine), exa.DeviceArray(ptr), exa.DeviceArray(it_run), levels)
+        if bad is None:
+            exa.volume_restriction_batch(*call)
+        else:
+            with pytest.raises(exa.ExaError):
+                exa.volume_restriction_batch(*call)
+        acc = coarse.copy()
+        for k, it in enumerate(items):
+            if k != bad:
+                acc[it[0]] = oracle.volume_unknowns_restriction(os_, acc[it[0]], fine[it[1]], 0, levels, it[2:])
+        assert _rel(d_acc.get(), acc) <= 1e-12
