@@ -59,19 +59,29 @@ def predictor_flops_ncp(B, V, D, picard_total, cells, c_s=ELASTIC_NCP_FLOPS):
     return per_iter * picard_total + fixed * cells
 
 
+def line_contraction_flops(B):
+    """FLOPs of one grid line's contraction by halves: B sums and differences of
+    the values, the even and the odd half (2 H^2 multiply-adds, H = B // 2; an
+    odd B adds H each for its middle node and its middle result) and B more
+    sums that put the results together."""
+    H = B // 2
+    return 4 * H * H + 4 * H + (4 * H if B % 2 else 0)
+
+
 def predictor_executed_flops_fp32(B, V, picard_total, cells):
     """FLOPs the default FP32-bulk predictor executes for a flux-only PDE (the
-    algorithmic count above counts every Picard iteration in full): the first
-    iteration evaluates one flux and one slice's Kxi contractions per node
-    (c_F + 6 V B) and forms lQi^1 in closed form and its residual (8 V B + 5 V);
-    later iterations are full; the epilogue adds the once-per-cell terms and,
-    except at B = 5, 6 and 8 where the flux averages are accumulated during
-    the iterations, re-evaluates the B slice fluxes of the last iterate
-    (c_F B^4)."""
+    algorithmic count above counts every Picard iteration and every contraction
+    in full): a slice's contractions are 3 V B^2 lines by halves; the first
+    iteration evaluates one flux and one slice's contractions and forms lQi^1
+    in closed form and its residual (8 V B + 5 V per node); later iterations
+    do so for B slices; the epilogue adds the once-per-cell terms and, except
+    at B = 5, 6 and 8 where the flux averages are accumulated during the
+    iterations, re-evaluates the B slice fluxes of the last iterate (c_F B^4)."""
     c_f = EULER_FLUX_FLOPS
-    first = B ** 3 * (c_f + 6 * V * B + 8 * V * B + 5 * V)
-    per_iter = 8 * V * B ** 5 + (c_f + 4 * V) * B ** 4
-    fixed = 2 * (3 * V + V) * B ** 4 + 12 * (V + V) * B ** 3 + 6 * V * B ** 4
+    slice_ = 3 * V * B * B * line_contraction_flops(B)
+    first = B ** 3 * (c_f + 8 * V * B + 5 * V) + slice_
+    per_iter = 2 * V * B ** 5 + B * slice_ + (c_f + 4 * V) * B ** 4
+    fixed = 2 * (3 * V + V) * B ** 4 + 12 * (V + V) * B ** 3 + slice_
     recompute = 0 if B in (5, 6, 8) else c_f * B ** 4
     return cells * first + (picard_total - cells) * per_iter + cells * (fixed + recompute)
 

@@ -395,7 +395,8 @@ struct exa_grid {
   double lo[3], hi[3], dx[3];
   bool periodic = true;
   int boundary = exa::kBoundaryPeriodic;
-  bool fused_corrector = true;  // Riemann + surface + update + dt in one kernel (nonlinear solvers)
+  // Riemann + surface + update + dt in one kernel (linear and user solvers: always)
+  bool fused_corrector = true;
   bool adjust = false;          // the PDE's adjust_point_solution after every update
   bool fused_ts = false;        // fused time stepping (fuse-algorithmic-steps)
   double fused_weight = 0.9;    // fuse-algorithmic-steps-factor

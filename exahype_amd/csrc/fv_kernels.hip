@@ -205,8 +205,9 @@ __device__ inline void atomic_max_positive(unsigned long long* slot, double v) {
 
 // The workgroup's eigenvalue maxima per direction into the state.  Atomics on
 // one address take 12 ns each whichever CU they come from, so a workgroup sends
-// one per direction, and none where the state already holds as much (a stale
-// value read here only costs the atomic): with one per wavefront they were the
+// one per direction, and none where the state already holds as much (the maxima
+// are reset in an earlier kernel and only grow within one, so a stale value is
+// too small and costs no more than the atomic): with one per wavefront they were the
 // longest part of a step on small grids (60x90x200 subcells 129 -> 62 us a step
 // with the tiles below) and of the stand-alone reductions (20 million subcells
 // 1.15 -> 0.18 ms).

@@ -54,9 +54,11 @@ enum { EXA_PRECISION_FP64 = 0, EXA_PRECISION_FP32_BULK = 1 };
 
 /* Space-time predictor variants (the device kernel behind
  * spaceTimePredictorNonlinear + volumeIntegralNonlinear).  AUTO: the default,
- * the tensor contractions on the vector ALUs with a 144 KB LDS budget for the
- * Picard iterate (measured fastest); VALU_LDS64 / VALU_LDS144: the vector-ALU
- * kernel with a 64 KB / 144 KB LDS budget; MFMA: the FP32-bulk form of the
+ * measured fastest: a thread per node with the contractions on the vector ALUs
+ * and a 144 KB LDS budget for the Picard iterate, or, for the Euler solvers
+ * without parameters at order 6, a wavefront per time slice; VALU_LDS64 /
+ * VALU_LDS144: the kernel with a thread per node and a 64 KB / 144 KB LDS
+ * budget; MFMA: the FP32-bulk form of the
  * Euler solvers (no parameters, orders 2..7) with the contractions on the
  * matrix cores (v_mfma_f32_4x4x1f32).  The variants compute the same
  * mathematics and differ in rounding order only. */
@@ -331,7 +333,8 @@ int exa_grid_set_predictor_variant(exa_grid* g, int variant);
  * and its neighbours' face blocks and applies surface integral, solution
  * update and the stable dt (the fluxes of a face are identical in both cells);
  * off: a face pass writing both cells' flux blocks, then the update pass.
- * Linear solvers always run the two passes (EXA_E_UNSUPPORTED for on). */
+ * Linear solvers have one form only, a single kernel that needs the face
+ * states and no fluxes: on is EXA_E_UNSUPPORTED, off changes nothing. */
 int exa_grid_set_fused_corrector(exa_grid* g, int on);
 /* Fused time stepping: the optimisation `fuse-algorithmic-steps` with
  * `fuse-algorithmic-steps-factor` weight in (0, 1] (Parser.cpp:486-505;

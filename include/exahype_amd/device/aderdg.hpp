@@ -238,9 +238,10 @@ enum : int { kPredictorAuto = 0, kPredictorValu64 = 1, kPredictorValu144 = 2, kP
 constexpr int kPredictorVariants = 4;
 // Bytes of PredictorArgs::ws one cell needs (0: no workspace), for a variant.
 size_t predictor_ws_bytes_per_cell(const SolverDesc& sd, int variant = kPredictorAuto);
-// Bit v set: variant v runs a kernel of its own for this solver (bit 0 always;
+// Bit v set: variant v is worth timing for this solver (bit 0 always;
 // kPredictorValu144 is the Auto kernel or the slower of the two, so its bit is
-// never set).
+// never set; kPredictorValu64 is the Auto kernel, too, where both budgets hold
+// the whole iterate: orders up to 4, and 5 in float).
 unsigned predictor_variants(const SolverDesc& sd);
 // Whether a variant can be requested for this solver (it may share Auto's kernel).
 bool predictor_variant_available(const SolverDesc& sd, int variant);

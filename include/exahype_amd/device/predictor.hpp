@@ -150,11 +150,12 @@ struct PredictorLayout {
 // Waves per SIMD the register allocation must leave room for: the float
 // flux-only form at N=5 and N=7 accumulates its time-averaged fluxes during
 // the last iteration (3V more live registers) within the four (N=5) or three
-// (N=7, 64 KB layout) waves that its LDS allows anyway; the elastic PDE, whose
-// next iterate alone takes 9 B registers or twice that, keeps the wavefronts
-// that its LDS allows (without the cap the compiler moves the line reads of
-// all variables to the front and one wavefront per SIMD is left); elsewhere no
-// constraint.
+// (N=7, 64 KB layout) waves that its LDS allows anyway; the library's elastic
+// PDE, whose next iterate alone takes 9 B registers or twice that, keeps the
+// wavefronts that its LDS allows (uncapped, N=4 in double takes 258 registers,
+// one wavefront per SIMD; in float 168 and 189 instead of 160 and 169 at N=4, 5).
+// By type, because the product of another PDE of these sizes may need more and
+// would spill; elsewhere no constraint.
 template <int B, class PDE, int TERMS, bool EXPORT, typename T>
 __host__ __device__ constexpr int predictor_min_waves() {
   if (std::is_same_v<PDE, Elastic>) return sizeof(T) == sizeof(double) ? (B <= 5 && !EXPORT ? 2 : 1) : (B <= 5 ? 3 : 2);
