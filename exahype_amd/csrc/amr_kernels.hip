@@ -26,12 +26,14 @@
 //   by workgroup: the lines of one transfer over up to four wavefronts, all
 //     levels' operators staged in LDS with the block;
 //   by value: one thread per value of the block, which stays in a register.
-// Bound: short lists by the chain item, block, passes, store; long ones by the
-// passes' LDS accesses and the stores of the fine blocks (a prolongation writes
-// every fine block once).  183,141 transfers of 6^3 x 5 values by wavefronts: the
-// prolongation 0.55 ms (2.9 TB/s), the restriction 0.68 ms (2.4 TB/s; its next
-// block is loaded while the last is restricted); with a thread per node and
-// B-term sums per node and pass 1.11 and 1.40.
+// Bound: the chain item, block, passes, store of a transfer, in short lists and
+// in long ones, where three to four wavefronts per SIMD spend more than half of
+// their time waiting (the LDS is busy in 45% of the cycles of a prolongation, VALU
+// instructions are active in 30%; a third of the LDS cycles are bank conflicts).
+// 183,141 transfers of 6^3 x 5 values by wavefronts: the prolongation 0.55 ms
+// (2.9 TB/s), the restriction 0.68 ms (2.4 TB/s; its next block is loaded while
+// the last is restricted); with a thread per node and B-term sums per node and
+// pass 1.11 and 1.40.
 #include "amr.hpp"
 #include "exa_device.hpp"
 

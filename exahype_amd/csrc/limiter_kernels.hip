@@ -320,8 +320,10 @@ __global__ __launch_bounds__(kLimNT) void lim_ghost_kernel(LimArgs a, int only_i
 // states are formed once, by the last wavefronts, beside the interior's
 // evolution.  So a patch takes 81 KB of LDS (N=3) and seven wavefronts, two
 // workgroups per CU within 128 registers; the states of all directions and both
-// sides took 147 KB, one workgroup per CU.  Bound by FP64 issue and the
-// barriers of a direction (three each).  Blast wave, one launch (MUSCL-Hancock):
+// sides took 147 KB, one workgroup per CU.  Half of a wavefront's time is
+// waiting, at the three barriers of a direction and on divides and roots; VALU
+// instructions are active in 48% of the SIMDs' cycles, the LDS is busy in 30%.
+// Blast wave, one launch (MUSCL-Hancock):
 //   N=3, 63x60x55 cells: 0.99 -> 0.50 ms;  N=2, 15^3 cells: 77 -> 39 us.
 // (A thread per evolved cell, ten wavefronts a patch: 0.86 ms and 54 us -- dealt
 // three to two SIMDs, a second workgroup of 96 registers does not fit.)
@@ -567,9 +569,9 @@ __global__ __launch_bounds__(MusclShape<N>::NT, (DT_MAX ? 2 : 4)) void lim_fv_up
 // lane (Y,X) forms out[Z][Y][X] for all Z and hands each value to
 // emit(Z, Y*M + X, value) in registers.  A lane reads its P inputs once for
 // M outputs, and the table index is uniform in every loop, so the table
-// entries are scalar loads from constant memory: the status kernel is bound
-// by LDS instruction issue, and an output per lane (P input and P table reads
-// each) took three times the LDS instructions.  Every output is the sum
+// entries are scalar loads from constant memory: an output per lane (P input
+// and P table reads each) took three times the LDS instructions, which then
+// bounded the status kernel.  Every output is the sum
 // 0 + in[0]*T[0][.] + ... + in[P-1]*T[P-1][.] of tensor3, in that order.
 enum { kTabUh2Lim, kTabUh2Lob, kTabLim2Uh };  // the table of tensor3_rows
 
@@ -624,9 +626,10 @@ constexpr int kStatusCells = 4;  // cells (wavefronts) per workgroup of the stat
 
 template <int N>
 // Registers capped for five wavefronts per SIMD (88 used at N=3); six spill.
-// FP64 issue and LDS both near their limits: 208,000 cells at N=3 1.02 -> 0.87
-// ms with the minima reduced by register moves, one instruction per minimum and
-// the extrema kept in LDS instead of selected into registers.
+// Bound by VALU issue: active in 74% of the SIMDs' cycles at N=3, the LDS busy
+// in 49% of the CUs'.  208,000 cells at N=3 1.02 -> 0.87 ms with the minima
+// reduced by register moves, one instruction per minimum and the extrema kept in
+// LDS instead of selected into registers.
 __global__ __launch_bounds__(kStatusCells * kWave, 5) void lim_update_status_kernel(LimArgs a) {
   using Sh = LimShape<N>;
   constexpr int B = Sh::B, B2 = B * B, B3 = Sh::B3, L = Sh::L, L3 = Sh::L3, V = Sh::V, PATCH = Sh::PATCH;
